@@ -192,6 +192,8 @@ void fill_params(dgsem_handle* h) {
   p.grad_out = h->d_grad;
   p.visc_out = h->d_visc;
   for (int k = 0; k < 3; ++k) p.cells[k] = c.cells[k];
+  p.div_y = dgsem::FastDiv::by((uint32_t)c.cells[1]);
+  p.div_z = dgsem::FastDiv::by((uint32_t)c.cells[2]);
   for (int f = 0; f < 6; ++f) {
     p.bc[f] = f < 2 * c.dim ? c.face_boundary[f] : dgsem::kBcPeriodic;
     for (int v = 0; v < 5; ++v) p.bc_state[f][v] = c.face_state[f][v];

@@ -391,6 +391,15 @@ bool box_metric_table(const Geometry& g, std::vector<double>& tab, int64_t off[3
   auto ja = [&](int64_t e, int dof, int r, int c) {
     return g.contravariant[((e * nn + dof) * d + r) * d + c];
   };
+  // position of node dof in a direction-r row: line * n + k, lines enumerating
+  // the remaining node indices in increasing dimension order
+  const int n = g.n;
+  auto line_pos = [&](int r, int dof) {
+    const int ix[3] = {dof % n, (dof / n) % n, dof / (n * n)};
+    if (d == 2) return ix[1 - r] * n + ix[r];
+    const int a = ix[r == 0 ? 1 : 0], b = ix[r == 2 ? 1 : 2];
+    return (b * n + a) * n + ix[r];
+  };
   // the rows of the elements with i_c = 0
   for (int64_t e = 0; e < E; ++e) {
     int eid[3];
@@ -399,7 +408,8 @@ bool box_metric_table(const Geometry& g, std::vector<double>& tab, int64_t off[3
       if (eid[c] != 0) continue;
       const int64_t pr = pair_of(eid, c);
       for (int r = 0; r < d; ++r)
-        for (int dof = 0; dof < nn; ++dof) tab[off[c] + (pr * d + r) * nn + dof] = ja(e, dof, r, c);
+        for (int dof = 0; dof < nn; ++dof)
+          tab[off[c] + (pr * d + r) * nn + line_pos(r, dof)] = ja(e, dof, r, c);
     }
   }
   // every element against its rows, bit for bit
@@ -412,7 +422,7 @@ bool box_metric_table(const Geometry& g, std::vector<double>& tab, int64_t off[3
       const int64_t pr = pair_of(eid, c);
       for (int r = 0; r < d; ++r)
         for (int dof = 0; dof < nn; ++dof) {
-          const double a = ja(e, dof, r, c), b = tab[off[c] + (pr * d + r) * nn + dof];
+          const double a = ja(e, dof, r, c), b = tab[off[c] + (pr * d + r) * nn + line_pos(r, dof)];
           uint64_t ua, ub;
           std::memcpy(&ua, &a, 8);
           std::memcpy(&ub, &b, 8);

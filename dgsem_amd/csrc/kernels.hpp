@@ -39,6 +39,24 @@ enum BoundaryKind : int {
   kBcMixedDirichletSlipWall = 6,  // per-node choice, states [node][NV + 1]
 };
 
+// Division of 0 <= x < 2^31 by a constant d >= 1 as a multiply-high and a
+// shift: with s = ceil(log2 d) and mul = floor(2^(31+s) / d) + 1, x / d is
+// x mul >> (31 + s): mul d = 2^(31+s) + r with 0 < r <= d <= 2^s, and x r <
+// 2^(31+s) keeps the excess below 1 / d.  A division by a run-time value takes
+// some twenty instructions otherwise.
+struct FastDiv {
+  uint32_t mul;
+  int32_t shift;
+  __host__ __device__ static FastDiv by(uint32_t d) {
+    int s = 0;
+    while ((1ull << s) < d) ++s;
+    return {(uint32_t)((1ull << (31 + s)) / d + 1), s};
+  }
+  __host__ __device__ int operator()(int x) const {
+    return (int)((uint32_t)((((uint64_t)(uint32_t)x << 1) * mul) >> 32) >> shift);
+  }
+};
+
 struct KParams {
   const double* u;       // stage input, [E][NV][NN]
   const double* u_base;  // base state for kModeStage3
@@ -49,10 +67,11 @@ struct KParams {
   // Box meshes (the linear mapping of a Cartesian box, nodal geometry): the
   // metric terms Ja^r_c of a node depend on its element only through the
   // element's indices in the directions other than c, so each distinct row
-  // is stored once: ja_box[ja_box_off[c] + (pair * DIM + r) * NN + dof] with
-  // pair = i_m * cells[l] + i_l (3D; m = c+1, l = c+2 mod 3) or i_m (2D;
-  // m = 1-c).  Null unless the mesh is such a box, whose 1/J is then
-  // positive at every node.
+  // is stored once: ja_box[ja_box_off[c] + (pair * DIM + r) * NN + line * n + k]
+  // with pair = i_m * cells[l] + i_l (3D; m = c+1, l = c+2 mod 3) or i_m (2D;
+  // m = 1-c), for node k of line `line` of direction r: the row a line thread
+  // reads is contiguous.  Null unless the mesh is such a box, whose 1/J is
+  // then positive at every node.
   const double* ja_box;
   int64_t ja_box_off[3];
   const double* Ja;      // nodal: [E][dim][dim][NN]; affine: [E][dim][dim]
@@ -81,6 +100,7 @@ struct KParams {
   // 0 = periodic, then nbr holds -1 at that face), constant Dirichlet states
   // and optional per-node Dirichlet states
   int cells[3];
+  FastDiv div_y, div_z;  // by cells[1] and cells[2]
   int bc[6];
   double bc_state[6][5];
   const double* bc_values[6];

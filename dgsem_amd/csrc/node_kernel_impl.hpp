@@ -281,7 +281,8 @@ __global__ void __launch_bounds__((Shape<DIM, N>::NN)) __attribute__((amdgpu_wav
   const int idx[3] = {a % n, (a / n) % n, DIM == 3 ? a / (n * n) : 0};
   constexpr int stride[3] = {1, n, n * n};
   const int pa = lds_pos<N>(a);
-  const int nz = DIM == 3 ? p.cells[2] : 1;
+  int eid[3];
+  element_indices<DIM>(p, (int)e, eid);
 
   // 1. the node's state, metric rows and 1/J (the face data follows the
   // term loops, phase 4)
@@ -432,7 +433,7 @@ __global__ void __launch_bounds__((Shape<DIM, N>::NN)) __attribute__((amdgpu_wav
       const bool lower = idx[d] == 0, upper = idx[d] == N;
       if (lower || upper) {
         int64_t lo, hi;
-        face_neighbours<DIM, false>(p, p.cells[0], p.cells[1], nz, e, d, lo, hi);
+        face_neighbours<DIM, false>(p, eid, e, d, lo, hi);
         const int64_t ve = lower ? e : hi;
         const int vn = lower ? a : a - N * stride[d];
         const double vij = lower ? ij : (NODAL ? p.invJ[ve * NN + vn] : p.invJ[ve]);
@@ -458,7 +459,7 @@ __global__ void __launch_bounds__((Shape<DIM, N>::NN)) __attribute__((amdgpu_wav
     const bool lower = idx[d] == 0, upper = idx[d] == N;
     if (lower || upper) {
       int64_t lo, hi;
-      face_neighbours<DIM, false>(p, p.cells[0], p.cells[1], nz, e, d, lo, hi);
+      face_neighbours<DIM, false>(p, eid, e, d, lo, hi);
       const int64_t ne = lower ? lo : hi;
       const int nn = lower ? a + N * stride[d] : a - N * stride[d];
       double un[NV], uo[NV], nrm[DIM], f[NV];

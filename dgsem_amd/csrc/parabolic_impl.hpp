@@ -378,7 +378,8 @@ __global__ void __launch_bounds__((Shape<DIM, N>::NN)) gradient_node_kernel(cons
   const int64_t e = xcd_block(blockIdx.x, gridDim.x);
   const int idx[3] = {a % n, (a / n) % n, DIM == 3 ? a / (n * n) : 0};
   constexpr int stride[3] = {1, n, n * n};
-  const int nz = DIM == 3 ? p.cells[2] : 1;
+  int eid[3];
+  element_indices<DIM>(p, (int)e, eid);
   double u[NV], q[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) u[v] = p.u[(e * NV + v) * NN + a];
@@ -422,7 +423,7 @@ __global__ void __launch_bounds__((Shape<DIM, N>::NN)) gradient_node_kernel(cons
     const bool lower = idx[d] == 0, upper = idx[d] == N;
     if (lower || upper) {
       int64_t lo, hi;
-      face_neighbours<DIM, false>(p, p.cells[0], p.cells[1], nz, e, d, lo, hi);
+      face_neighbours<DIM, false>(p, eid, e, d, lo, hi);
       const int64_t ne = lower ? lo : hi;
       const int nn = lower ? a + N * stride[d] : a - N * stride[d];
       double un[NV], qn[NV], nrm[DIM];

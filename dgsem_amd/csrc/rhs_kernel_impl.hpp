@@ -55,19 +55,22 @@ __device__ __forceinline__ int lds_pos(int node) {
   return node + node / (N + 1);
 }
 
-// Metric term Ja^r_c at node `dof` of the element with indices eid on a box
-// mesh, from the table described at KParams::ja_box.
+// The row of metric terms Ja^r_c, c fixed, of line `line` (n nodes) of the
+// element with indices eid on a box mesh, in the table described at
+// KParams::ja_box.
 template <int DIM, int N>
-__device__ __forceinline__ double box_ja(const KParams& p, const int* eid, int c, int r, int dof) {
-  constexpr int NN = Shape<DIM, N>::NN;
-  int64_t pair;
+__device__ __forceinline__ const double* box_row(const KParams& p, const int* eid, int c, int r,
+                                                 int line) {
+  constexpr int NN = Shape<DIM, N>::NN, n = N + 1;
+  // pairs <= E < 2^30 (the ABI's limit): 32 bits hold the row index
+  uint32_t pair;
   if constexpr (DIM == 3) {
     const int m = c == 2 ? 0 : c + 1, l = c == 0 ? 2 : c - 1;  // (c + 1) % 3, (c + 2) % 3
-    pair = (int64_t)eid[m] * p.cells[l] + eid[l];
+    pair = (uint32_t)eid[m] * (uint32_t)p.cells[l] + (uint32_t)eid[l];
   } else {
-    pair = eid[1 - c];
+    pair = (uint32_t)eid[1 - c];
   }
-  return p.ja_box[p.ja_box_off[c] + (pair * DIM + r) * NN + dof];
+  return p.ja_box + p.ja_box_off[c] + (uint64_t)(pair * DIM + r) * NN + line * n;
 }
 
 // Elements per workgroup: keeps EPW * LINES near 192 threads.
@@ -93,6 +96,45 @@ __device__ __forceinline__ int line_dof(int dir, int line, int k) {
   }
 }
 
+// The nodes of line `line` of direction dir: node k is dof base + k stride, at
+// the padded LDS position pbase + k pstride.  Every value is an arithmetic
+// select of the direction, so a thread sets its line up without branches;
+// per-node calls of line_dof compile to a branch each, and with the run-time
+// integer divisions of the element indices they had made up a third of the
+// 3D N = 3 kernel's instructions (with them out, and whole-node staging, the
+// SSPRK3 step at 64^3 N = 3 went from 2.34 to 2.12 ms, the warped 27 x 19 x 22
+// N = 4 right-hand side from 219 to 197 us).
+template <int DIM, int N>
+struct LineNodes {
+  int base, stride, pbase, pstride;
+  __device__ __forceinline__ LineNodes(int dir, int line) {
+    constexpr int n = N + 1;
+    if constexpr (DIM == 2) {
+      base = dir == 0 ? line * n : line;
+      stride = dir == 0 ? 1 : n;
+      pbase = dir == 0 ? line * (n + 1) : line;
+      pstride = dir == 0 ? 1 : n + 1;
+    } else {
+      const int b = line / n, a = line - b * n;
+      const int row = dir == 0 ? line : (dir == 1 ? b * n : b);  // row of the line's first node
+      const int i = dir == 0 ? 0 : a;                            // its place in that row
+      base = row * n + i;
+      pbase = row * (n + 1) + i;
+      stride = dir == 0 ? 1 : (dir == 1 ? n : n * n);
+      pstride = dir == 0 ? 1 : (dir == 1 ? n + 1 : n * (n + 1));
+    }
+  }
+};
+
+// Indices of element e on the structured grid, e = (ie * ny + je) * nz + ke.
+template <int DIM>
+__device__ __forceinline__ void element_indices(const KParams& p, int e, int* id) {
+  const int t = DIM == 3 ? p.div_z(e) : e;
+  id[2] = DIM == 3 ? e - t * p.cells[2] : 0;
+  id[0] = p.div_y(t);
+  id[1] = t - id[0] * p.cells[1];
+}
+
 // Maps hardware block ids (dispatched round-robin over the 8 XCDs) to
 // contiguous element ranges per XCD, so face neighbours share an L2.
 __device__ __forceinline__ int xcd_block(int b, int nb) {
@@ -108,30 +150,26 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
 // The modal coefficients come from one sweep of V^-1 per direction.  A
 // sweep gives each thread one line of n nodes (EPW n^(DIM-1) lines), so every
 // index into V^-1 is a compile-time constant and its entries are scalar
-// loads; the first sweep forms the indicator variable of its line's nodes
-// itself.  Each output is the sum over the line in increasing order, with
+// loads.  Each output is the sum over the line in increasing order, with
 // the same fused multiply-adds as a node-parallel sweep.  A thread reads its
 // line before it writes it, so every sweep works in place in one scratch
 // plane per element, at the padded node positions of the state planes
 // (lds_pos): the line reads and writes hit distinct banks.  The energy sums
-// follow the reference's order, one thread per element.
-//
-// OVERLAP: the sweeps and the energy sums keep only EPW n^(DIM-1) and EPW
-// threads busy; the others meanwhile form the per-node primitives, prim(i)
-// for i < EPW NN, a slice per phase.  s_w (indicator_scratch() doubles) then
-// lies apart from the primitives' array; without OVERLAP it may be that
-// array, and prim goes unused.
+// follow the reference's order, one thread per element.  s_w holds the
+// indicator variable of every node on entry (indicator_scratch() doubles).
 template <int DIM, int N, int EPW>
 constexpr int indicator_scratch() {
   return EPW * Shape<DIM, N>::PN;
 }
 
-// Whether a shock-capturing kernel overlaps the primitives with the
-// indicator: only where its separate scratch leaves the LDS-bound number of
-// blocks per CU (160 KiB of LDS) unchanged -- in 2D at N = 3 it would cut
-// three blocks to two, and the step measured 23% slower.
+// Whether a shock-capturing kernel gives the indicator its own scratch, so
+// that the primitives are formed while the state is staged: only where that
+// leaves the LDS-bound number of blocks per CU (160 KiB of LDS) unchanged --
+// in 2D at N = 3 it would cut three blocks to two, and the step measured 23%
+// slower.  Otherwise the scratch is the primitives' array, and they follow
+// the indicator.
 template <int DIM, int N, int EPW, bool SC>
-constexpr bool overlap_prims() {
+constexpr bool separate_indicator() {
   using S = Shape<DIM, N>;
   constexpr int lds_cu = 160 * 1024;
   constexpr int base = 8 * (EPW * (S::SU + S::SP) + EPW);
@@ -139,39 +177,22 @@ constexpr bool overlap_prims() {
   return SC && lds_cu / with == lds_cu / base;
 }
 
-template <int DIM, int N, int EPW, int BLOCK, bool OVERLAP, class Prim>
-__device__ void block_alpha(const KParams& p, const double* s_u, double* s_w, double* s_alpha,
-                            int nvalid, Prim&& prim) {
+template <int DIM, int N, int EPW, int BLOCK>
+__device__ void block_alpha(const KParams& p, double* s_w, double* s_alpha, int nvalid) {
   using S = Shape<DIM, N>;
-  constexpr int n = S::n, NN = S::NN, NV = S::NV, PN = S::PN;
-  constexpr int LN = NN / n;    // lines per direction and element
-  constexpr int T0 = EPW * LN;  // threads of a sweep
-  static_assert(!OVERLAP || T0 < BLOCK, "threads left for the primitives");
-  static_assert(OVERLAP || indicator_scratch<DIM, N, EPW>() <= EPW * S::SP,
+  constexpr int n = S::n, NN = S::NN, PN = S::PN;
+  constexpr int LN = NN / n;  // lines per direction and element
+  static_assert(indicator_scratch<DIM, N, EPW>() <= EPW * S::SP,
                 "indicator scratch in the primitives' LDS");
-  constexpr int PHASES = DIM + 1;  // the sweeps and the energy sums
   double* A = s_w;
   const double* V = p.Vinv;
   const int tid = threadIdx.x;
-  // the primitives' slice of phase f, on the threads a sweep leaves idle
-  auto prims_slice = [&](int f) {
-    if (OVERLAP && tid >= T0) {
-      const int lo = f * (EPW * NN) / PHASES, hi = (f + 1) * (EPW * NN) / PHASES;
-      for (int i = lo + (tid - T0); i < hi; i += BLOCK - T0) prim(i);
-    }
-  };
-  // sweep along xi, lines of fixed (j, k), from the indicator variable
-  prims_slice(0);
+  // sweep along xi, lines of fixed (j, k)
   for (int t = tid; t < EPW * LN; t += BLOCK) {
     const int slot = t / LN, row = (t % LN) * n;  // the line's node i = 0
     double x[n];
 #pragma unroll
-    for (int ii = 0; ii < n; ++ii) {
-      double s[NV];
-#pragma unroll
-      for (int v = 0; v < NV; ++v) s[v] = s_u[slot * S::SU + v * PN + lds_pos<N>(row + ii)];
-      x[ii] = slot < nvalid ? indicator_variable<DIM>(s) : 0.0;
-    }
+    for (int ii = 0; ii < n; ++ii) x[ii] = A[slot * PN + lds_pos<N>(row + ii)];
 #pragma unroll
     for (int i = 0; i < n; ++i) {
       double r = 0.0;
@@ -182,7 +203,6 @@ __device__ void block_alpha(const KParams& p, const double* s_u, double* s_w, do
   }
   __syncthreads();
   // sweep along eta, lines of fixed (i, k)
-  prims_slice(1);
   for (int t = tid; t < EPW * LN; t += BLOCK) {
     const int slot = t / LN, l = t % LN;
     const int base = (l / n) * n * n + l % n;
@@ -201,7 +221,6 @@ __device__ void block_alpha(const KParams& p, const double* s_u, double* s_w, do
   const double* modal = A;
   if constexpr (DIM == 3) {
     // sweep along zeta, lines of fixed (i, j)
-    prims_slice(2);
     for (int t = tid; t < EPW * LN; t += BLOCK) {
       const int slot = t / LN, base = t % LN;
       double x[n];
@@ -217,7 +236,6 @@ __device__ void block_alpha(const KParams& p, const double* s_u, double* s_w, do
     }
     __syncthreads();
   }
-  prims_slice(DIM);
   if (tid < nvalid) {
     const double* m = modal + tid * PN;
     auto M = [&](int k, int j, int i) { return m[lds_pos<N>((k * n + j) * n + i)]; };
@@ -285,16 +303,15 @@ constexpr bool pair_fence() {
 // structured grid of cells[] (element index (ie * ny + je) * nz + ke): the
 // periodic wrap, or -1 at a non-periodic boundary face (BCS: kinds from
 // p.bc) -- what the neighbour table holds, computed rather than loaded so
-// that the neighbour traces do not wait on a dependent load.  The grid
-// sizes come in as values: selecting them per thread from the parameter
-// block would index it dynamically and turn the reads into vector loads.
+// that the neighbour traces do not wait on a dependent load.  id: the
+// element's indices (element_indices).
 template <int DIM, bool BCS>
-__device__ __forceinline__ void face_neighbours(const KParams& p, int nx, int ny, int nz, int64_t e,
-                                                int dir, int64_t& lo, int64_t& hi) {
-  const int ei = (int)e;
+__device__ __forceinline__ void face_neighbours(const KParams& p, const int* id, int64_t e, int dir,
+                                                int64_t& lo, int64_t& hi) {
+  const int nx = p.cells[0], ny = p.cells[1], nz = DIM == 3 ? p.cells[2] : 1;
   const int stride = dir == 0 ? ny * nz : (dir == 1 ? nz : 1);
   const int count = dir == 0 ? nx : (dir == 1 ? ny : nz);
-  const int idx = dir == 0 ? ei / stride : (dir == 1 ? (ei / nz) % ny : ei % nz);
+  const int idx = dir == 0 ? id[0] : (dir == 1 ? id[1] : id[2]);
   bool wrap_lo = true, wrap_hi = true;
   if constexpr (BCS) {
     const int blo = dir == 0 ? p.bc[0] : (dir == 1 ? p.bc[2] : p.bc[4]);
@@ -302,8 +319,15 @@ __device__ __forceinline__ void face_neighbours(const KParams& p, int nx, int ny
     wrap_lo = blo == kBcPeriodic;
     wrap_hi = bhi == kBcPeriodic;
   }
-  lo = idx > 0 ? e - stride : (wrap_lo ? e + (int64_t)(count - 1) * stride : -1);
-  hi = idx < count - 1 ? e + stride : (wrap_hi ? e - (int64_t)(count - 1) * stride : -1);
+  // E < 2^30 (the ABI's limit), so 32-bit element arithmetic suffices
+  const int ei = (int)e, wrap = (count - 1) * stride;
+  int l = ei + (idx > 0 ? -stride : wrap), h = ei + (idx < count - 1 ? stride : -wrap);
+  if constexpr (BCS) {
+    if (!wrap_lo && idx == 0) l = -1;
+    if (!wrap_hi && idx == count - 1) h = -1;
+  }
+  lo = l;
+  hi = h;
 }
 
 // Outer state of a non-periodic face of a 2D compressible-Euler mesh, seen
@@ -378,8 +402,9 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES))
   __shared__ double s_u[EPW * S::SU];
   __shared__ double s_p[EPW * S::SP];
   __shared__ double s_alpha[EPW];
-  constexpr bool OVERLAP = overlap_prims<DIM, N, EPW, SC>();
-  __shared__ double s_ind[OVERLAP ? indicator_scratch<DIM, N, EPW>() : 1];
+  constexpr bool SEP = separate_indicator<DIM, N, EPW, SC>();
+  __shared__ double s_ind_own[SEP ? indicator_scratch<DIM, N, EPW>() : 1];
+  double* const s_ind = SEP ? s_ind_own : s_p;
   double* const s_du = s_p;
 
   const int tid = threadIdx.x;
