@@ -41,6 +41,10 @@ constexpr int ad_elems_per_block() {
   return e < 1 ? 1 : e;
 }
 
+// Planes of the node primitives rho, v[DIM], beta, kin, p, c.
+template <int DIM>
+constexpr int kAdPrims = DIM + 5;
+
 __device__ __forceinline__ double combine(const AdParams& a, int64_t g, double r) {
   double o = a.c * r;
   if (a.b != 0.0) o += a.b * a.v[g];
@@ -396,7 +400,7 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) jvp_visc_kernel(
 template <int DIM, int N, int EPW, bool NODAL, bool NS, bool SC, int SF, int FF>
 __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) jvp_rhs_kernel(const AdParams a) {
   using S = Shape<DIM, N>;
-  constexpr int n = S::n, NV = S::NV, NN = S::NN, FN = S::FN, L = S::LINES, NP = S::NP;
+  constexpr int n = S::n, NV = S::NV, NN = S::NN, FN = S::FN, L = S::LINES, NP = kAdPrims<DIM>;
   constexpr int NQ = DIM + 3;
   constexpr int BLOCK = EPW * L;
   const KParams& p = a.k;
@@ -811,14 +815,14 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) vjp_visc2_kernel
 template <int DIM, int N, int EPW, bool SC>
 constexpr bool par_subcell_adjoint() {
   using S = Shape<DIM, N>;
-  constexpr int lds = 8 * EPW * S::NN * (S::NP + 2 * S::NV + DIM + 3 + DIM * S::NV);
+  constexpr int lds = 8 * EPW * S::NN * (kAdPrims<DIM> + 2 * S::NV + DIM + 3 + DIM * S::NV);
   return SC && DIM == 3 && N <= 3 && lds <= 80 * 1024;
 }
 
 template <int DIM, int N, int EPW, bool NODAL, bool NS, bool SC, int SF, int FF>
 __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) vjp_rhs_kernel(const AdParams a) {
   using S = Shape<DIM, N>;
-  constexpr int n = S::n, NV = S::NV, NN = S::NN, FN = S::FN, L = S::LINES, NP = S::NP;
+  constexpr int n = S::n, NV = S::NV, NN = S::NN, FN = S::FN, L = S::LINES, NP = kAdPrims<DIM>;
   constexpr int NQ = DIM + 3;
   constexpr int BLOCK = EPW * L;
   const KParams& p = a.k;

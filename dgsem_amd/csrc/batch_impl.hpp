@@ -46,14 +46,10 @@ __device__ __forceinline__ void batch_tile(const KParams& p, const int64_t e0, c
   constexpr int PN = S::PN;
   constexpr int EPW = BLOCK / L;
   static_assert(EPW >= 1, "workgroup too small for one element");
-  static_assert(NP >= NV && NP >= 2, "s_p must be able to hold s_du and scratch");
+  static_assert(NP >= NV, "s_p must be able to hold s_du");
   double* const s_u = smem;
   double* const s_p = smem + EPW * S::SU;
   double* const s_alpha = s_p + EPW * S::SP;
-  // the indicator works in s_p, before the primitives: the LDS is sized for
-  // the largest degree of the ensemble, and 2D kernels are LDS-bound
-  constexpr bool SEP = false;
-  double* const s_ind = s_p;
   double* const s_du = s_p;
   // The thread's roles (line, direction, node positions) do not change from
   // tile to tile; computed from a plain threadIdx.x the compiler would hoist

@@ -409,7 +409,7 @@ bool box_metric_table(const Geometry& g, std::vector<double>& tab, int64_t off[3
       const int64_t pr = pair_of(eid, c);
       for (int r = 0; r < d; ++r)
         for (int dof = 0; dof < nn; ++dof)
-          tab[off[c] + (pr * d + r) * nn + line_pos(r, dof)] = ja(e, dof, r, c);
+          tab[off[c] + (pr * d + r) * nn + line_pos(r, dof)] = 0.5 * ja(e, dof, r, c);
     }
   }
   // every element against its rows, bit for bit
@@ -422,7 +422,7 @@ bool box_metric_table(const Geometry& g, std::vector<double>& tab, int64_t off[3
       const int64_t pr = pair_of(eid, c);
       for (int r = 0; r < d; ++r)
         for (int dof = 0; dof < nn; ++dof) {
-          const double a = ja(e, dof, r, c), b = tab[off[c] + (pr * d + r) * nn + line_pos(r, dof)];
+          const double a = 0.5 * ja(e, dof, r, c), b = tab[off[c] + (pr * d + r) * nn + line_pos(r, dof)];
           uint64_t ua, ub;
           std::memcpy(&ua, &a, 8);
           std::memcpy(&ub, &b, 8);

@@ -65,7 +65,7 @@ struct KParams {
   const double* alpha_in;  // [E] frozen blending factor to use instead of the
                            // indicator's (shock capturing), or null
   // Box meshes (the linear mapping of a Cartesian box, nodal geometry): the
-  // metric terms Ja^r_c of a node depend on its element only through the
+  // halved metric terms Ja^r_c / 2 of a node depend on its element only through the
   // element's indices in the directions other than c, so each distinct row
   // is stored once: ja_box[ja_box_off[c] + (pair * DIM + r) * NN + line * n + k]
   // with pair = i_m * cells[l] + i_l (3D; m = c+1, l = c+2 mod 3) or i_m (2D;

