@@ -15,7 +15,11 @@
 // thread holds only its node's five sums and one partner, so the kernel
 // fits four waves per SIMD with two elements per CU, and there is no
 // cross-thread accumulation: the node's result goes straight from registers
-// to memory.
+// to memory.  It is bound by instruction issue (the pair fluxes), so what it
+// saves is instructions: the shared reciprocals of the pair flux, the face
+// fluxes on fully active waves and the staged viscous terms took the 32^3 step
+// from 6.72 to 5.02 ms and the 24^3 Navier-Stokes step from 5.61 to 4.12 ms
+// (one MI355X), with the same bits.
 //
 // At N = 7 the split-form sums cancel terms some thousand times larger than
 // their result, so the RHS carries the last bits of every term and the
@@ -53,48 +57,58 @@ constexpr bool use_node_kernel() {
 // show in the RHS at the 1e-12 level; with the reference's roundings and its
 // summation order the kernel reproduces its results.
 
-// a / b rounded to nearest for positive normal operands, in fewer
-// instructions than the IEEE division sequence (which also scales for
-// denormal and overflowing operands): the hardware reciprocal estimate with
-// two Newton steps, the quotient, and one correction by its exact residual
-// (Markstein's method).  Equal to a / b on 2e8 random operand pairs.
-__device__ __forceinline__ double div_rn(double a, double b) {
-  double y = __builtin_amdgcn_rcp(b);
-  double e = fma(-b, y, 1.0);
-  y = fma(y, e, y);
-  e = fma(-b, y, 1.0);
-  y = fma(y, e, y);
-  const double q = a * y;
-  return fma(fma(-b, q, a), y, q);
-}
+// Quotients are div_by (physics.hpp): the estimate a y, y within 5e-14 of 1 / b,
+// corrected by its residual, which leaves less than 2e-11 of an ulp before the
+// final rounding.  A quotient then costs three instructions beside its share of
+// a reciprocal, against eleven for the IEEE sequence, with the same bits.
 
 // Sums below run left to right from their first term, as the reference's
 // written-out expressions do ((a + b) + c), in 2D and 3D alike.
 
-// rho, v, beta = rho / (2 p), |v|^2 / 2, p and c of a conservative state.
+// rho, v, beta = rho / (2 p), |v|^2 / 2 and p of a conservative state.
 template <int DIM>
 __device__ __forceinline__ NodePrims<DIM> node_prims_exact(double g, const double* u) {
 #pragma clang fp contract(off)
   NodePrims<DIM> q;
+  const double y = recip(u[0]);
   q.rho = u[0];
 #pragma unroll
-  for (int k = 0; k < DIM; ++k) q.v[k] = u[k + 1] / u[0];
+  for (int k = 0; k < DIM; ++k) q.v[k] = div_by(u[k + 1], u[0], y);
   double v2 = q.v[0] * q.v[0];
 #pragma unroll
   for (int k = 1; k < DIM; ++k) v2 = v2 + q.v[k] * q.v[k];
   q.kin = 0.5 * v2;
   q.p = (g - 1.0) * (u[DIM + 1] - 0.5 * u[0] * v2);
-  q.beta = 0.5 * u[0] / q.p;
-  q.c = sqrt(g * q.p / u[0]);
+  q.beta = div_by(0.5 * u[0], q.p, recip(q.p));
+  q.c = 0.0;  // not needed per node
   return q;
+}
+
+// A node of the pair flux: rho / 4, v, beta / 2 and |v|^2 / 2.  Scaling by a
+// power of two is exact, so the halvings of the reference's expressions move
+// into the stored values and drop out of the flux.
+template <int DIM>
+struct PairNode {
+  double r, v[DIM], b, kin;
+};
+
+// Logarithmic mean of lo <= hi by the reference's quotient.
+__device__ __forceinline__ double log_mean_exact(double x, double y) {
+  const double lo = dmin(x, y), hi = dmax(x, y);
+  return (hi - lo) / log(hi / lo);
 }
 
 // Chandrashekar flux, symmetric in (a, b) to the bit: the series test uses
 // ((x - y) / (x + y))^2 (whose rounding cannot reach the polynomial, which
 // is 2 to within 1e-4), and the log branch orders its arguments by value.
+// One reciprocal, of s_rho s_beta, serves the two ratios and both quotients by
+// s_beta; the reciprocal of a polynomial 1 + f2 / 3 + ... comes from its own
+// series.  88 FP64 issue slots a pair, against 125 with a reciprocal estimate
+// and refinement for each of the five quotients.  The last component is twice
+// the energy flux: its weight takes the half.
 template <int DIM>
-__device__ __forceinline__ void flux_chandrashekar_exact(double inv_gm1, const NodePrims<DIM>& a,
-                                                         const NodePrims<DIM>& b, const double* n,
+__device__ __forceinline__ void flux_chandrashekar_exact(double inv_gm1, const PairNode<DIM>& a,
+                                                         const PairNode<DIM>& b, const double* n,
                                                          double* f) {
 #pragma clang fp contract(off)
   double vna = a.v[0] * n[0], vnb = b.v[0] * n[0];
@@ -103,33 +117,39 @@ __device__ __forceinline__ void flux_chandrashekar_exact(double inv_gm1, const N
     vna = vna + a.v[k] * n[k];
     vnb = vnb + b.v[k] * n[k];
   }
-  const double sr = a.rho + b.rho, sb = a.beta + b.beta;
-  const double xr = a.rho - b.rho, xb = a.beta - b.beta;
-  const double r1 = recip((sr * sr) * (sb * sb));
-  const double f2r = (xr * xr) * ((sb * sb) * r1), f2b = (xb * xb) * ((sr * sr) * r1);
-  double rho_mean, beta_mean;
-  if (f2r < 1.0e-4) {
-    rho_mean = div_rn(sr, 2.0 + f2r * (2.0 / 3.0 + f2r * (2.0 / 5.0 + f2r * (2.0 / 7.0))));
+  const double sr = a.r + b.r, sb = a.b + b.b;  // s_rho / 4, s_beta / 2
+  const double rc = recip(sr * sb);
+  const double ysb = rc * sr;  // 2 / s_beta
+  const double xr = (a.r - b.r) * (rc * sb), xb = (a.b - b.b) * ysb;
+  const double f2r = xr * xr, f2b = xb * xb;
+  double q, gb;  // rho_mean / 2 and 1 / ((gamma - 1) beta_mean)
+  if (f2r < 1.0e-4 && f2b < 1.0e-4) {
+    // s_rho / (2 + 2/3 f2 + ...) over 4, 2 and 2
+    const double pr = fma(f2r, fma(f2r, fma(f2r, 1.0 / 7.0, 1.0 / 5.0), 1.0 / 3.0), 1.0);
+    const double pb = fma(f2b, fma(f2b, fma(f2b, 1.0 / 7.0, 1.0 / 5.0), 1.0 / 3.0), 1.0);
+    const double yr = fma(f2r, fma(f2r, -4.0 / 45.0, -1.0 / 3.0), 1.0);  // 1 / pr to 5e-14
+    const double yb = fma(f2b, fma(f2b, -4.0 / 45.0, -1.0 / 3.0), 1.0);
+    q = div_by(sr, pr, yr);
+    const double bm = div_by(sb, pb, yb);
+    gb = div_by(inv_gm1, bm, pb * ysb);
   } else {
-    const double lo = dmin(a.rho, b.rho), hi = dmax(a.rho, b.rho);
-    rho_mean = (hi - lo) / log(hi / lo);
+    const double pr = fma(f2r, fma(f2r, fma(f2r, 1.0 / 7.0, 1.0 / 5.0), 1.0 / 3.0), 1.0);
+    const double pb = fma(f2b, fma(f2b, fma(f2b, 1.0 / 7.0, 1.0 / 5.0), 1.0 / 3.0), 1.0);
+    q = f2r < 1.0e-4 ? sr / pr : 2.0 * log_mean_exact(a.r, b.r);
+    const double bm = f2b < 1.0e-4 ? sb / pb : 2.0 * log_mean_exact(a.b, b.b);
+    gb = inv_gm1 / bm;
   }
-  if (f2b < 1.0e-4) {
-    beta_mean = div_rn(sb, 2.0 + f2b * (2.0 / 3.0 + f2b * (2.0 / 5.0 + f2b * (2.0 / 7.0))));
-  } else {
-    const double lo = dmin(a.beta, b.beta), hi = dmax(a.beta, b.beta);
-    beta_mean = (hi - lo) / log(hi / lo);
-  }
-  const double p_mean = div_rn(0.5 * sr, sb);
+  const double p_mean = div_by(sr, sb, ysb);
   const double vsq = a.kin + b.kin;
-  const double f1 = rho_mean * 0.5 * (vna + vnb);
-  double fe = f1 * 0.5 * (div_rn(inv_gm1, beta_mean) - vsq);
+  const double f1 = q * (vna + vnb);
+  const double h = 0.5 * f1;
+  double fe = f1 * (gb - vsq);
   f[0] = f1;
 #pragma unroll
   for (int k = 0; k < DIM; ++k) {
-    const double vavg = 0.5 * (a.v[k] + b.v[k]);
-    f[k + 1] = f1 * vavg + p_mean * n[k];
-    fe = fe + f[k + 1] * vavg;
+    const double vs = a.v[k] + b.v[k];
+    f[k + 1] = h * vs + p_mean * n[k];
+    fe = fe + f[k + 1] * vs;
   }
   f[DIM + 1] = fe;
 }
@@ -142,8 +162,9 @@ __device__ __forceinline__ double physical_flux_exact(double g, const double* u,
 #pragma clang fp contract(off)
   constexpr int NV = DIM + 2;
   double v[DIM];
+  const double y = recip(u[0]);
 #pragma unroll
-  for (int k = 0; k < DIM; ++k) v[k] = u[k + 1] / u[0];
+  for (int k = 0; k < DIM; ++k) v[k] = div_by(u[k + 1], u[0], y);
   double v2 = v[0] * v[0];
 #pragma unroll
   for (int k = 1; k < DIM; ++k) v2 = v2 + v[k] * v[k];
@@ -173,10 +194,11 @@ __device__ __forceinline__ void flux_llf_exact(double g, const double* ul, const
   for (int s = 0; s < 2; ++s) {
     const double* u = s == 0 ? ul : ur;
     const double p = physical_flux_exact<DIM>(g, u, n, s == 0 ? fl : fr);
-    a[s] = sqrt(g * p / u[0]);
-    double vnn = (u[1] / u[0]) * n[0];
+    const double y = recip(u[0]);
+    a[s] = sqrt(div_by(g * p, u[0], y));
+    double vnn = div_by(u[1], u[0], y) * n[0];
 #pragma unroll
-    for (int k = 1; k < DIM; ++k) vnn = vnn + (u[k + 1] / u[0]) * n[k];
+    for (int k = 1; k < DIM; ++k) vnn = vnn + div_by(u[k + 1], u[0], y) * n[k];
     vn[s] = vnn;
   }
   double nn2 = n[0] * n[0];
@@ -203,11 +225,12 @@ __device__ __forceinline__ void flux_hllc_exact(double g, const double* ul, cons
 #pragma unroll
   for (int d = 0; d < DIM; ++d) nh[d] = n[d] / nrm;
   const double rho_ll = ul[0], rho_rr = ur[0], rhoE_ll = ul[NV - 1], rhoE_rr = ur[NV - 1];
+  const double yl = recip(rho_ll), yr = recip(rho_rr);
   double v2l = 0.0, v2r = 0.0, vn_l = 0.0, vn_r = 0.0;
 #pragma unroll
   for (int d = 0; d < DIM; ++d) {
-    vl[d] = ul[d + 1] / rho_ll;
-    vr[d] = ur[d + 1] / rho_rr;
+    vl[d] = div_by(ul[d + 1], rho_ll, yl);
+    vr[d] = div_by(ur[d + 1], rho_rr, yr);
     v2l += vl[d] * vl[d];
     v2r += vr[d] * vr[d];
     vn_l += vl[d] * nh[d];
@@ -271,8 +294,18 @@ __global__ void __launch_bounds__((Shape<DIM, N>::NN)) __attribute__((amdgpu_wav
   constexpr int PN = NN + NN / n;  // padded plane (lds_pos)
   constexpr int DS = n + 1;        // padded row of the D_split table
   constexpr int QB = DIM + 1;      // plane of beta; kin follows
-  __shared__ double s_q[(DIM + 3) * PN];             // rho, v[DIM], beta, kin
-  __shared__ double s_ja[NODAL ? DIM * DIM * PN : 1];  // Ja^d_c / 2
+  constexpr int FN = Shape<DIM, N>::FN;
+  constexpr int FACE = 2 * DIM * FN;  // face fluxes of the element, one per line end
+  // LDS planes: rho, v[DIM], beta, kin, then (NODAL) Ja^d_c / 2.  Once the term
+  // loops are done with them they take the face fluxes (FPL planes) and the
+  // viscous fluxes (VPL planes: the mass component is zero).
+  constexpr int QPL = DIM + 3, FPL = (FACE * NV + PN - 1) / PN, VPL = DIM * (NV - 1);
+  constexpr int JPL = NODAL ? DIM * DIM : 0;
+  constexpr int PLANES = QPL + JPL > FPL + VPL ? QPL + JPL : FPL + VPL;
+  __shared__ double s_q[PLANES * PN];
+  double* const s_ja = s_q + QPL * PN;
+  double* const s_face = s_q;                 // [dir][side][var][line]
+  double* const s_vf = s_q + FPL * PN;        // [dir][var - 1][node], padded
   __shared__ double s_D[n * DS];
   __shared__ double s_Dh[n * DS];  // D_hat (Navier-Stokes viscous terms)
 
@@ -299,11 +332,17 @@ __global__ void __launch_bounds__((Shape<DIM, N>::NN)) __attribute__((amdgpu_wav
 
   // 2. the node's primitives and halved metric rows into LDS
   const NodePrims<DIM> q = node_prims_exact<DIM>(p.gamma, u);
-  s_q[pa] = q.rho;
+  PairNode<DIM> qa;  // scaled as the flux takes it
+  qa.r = 0.25 * q.rho;
 #pragma unroll
-  for (int c = 0; c < DIM; ++c) s_q[(1 + c) * PN + pa] = q.v[c];
-  s_q[QB * PN + pa] = q.beta;
-  s_q[(QB + 1) * PN + pa] = q.kin;
+  for (int c = 0; c < DIM; ++c) qa.v[c] = q.v[c];
+  qa.b = 0.5 * q.beta;
+  qa.kin = q.kin;
+  s_q[pa] = qa.r;
+#pragma unroll
+  for (int c = 0; c < DIM; ++c) s_q[(1 + c) * PN + pa] = qa.v[c];
+  s_q[QB * PN + pa] = qa.b;
+  s_q[(QB + 1) * PN + pa] = qa.kin;
   if constexpr (NODAL) {
 #pragma unroll
     for (int d = 0; d < DIM; ++d)
@@ -327,61 +366,118 @@ __global__ void __launch_bounds__((Shape<DIM, N>::NN)) __attribute__((amdgpu_wav
   double acc[NV];
 #pragma unroll
   for (int v = 0; v < NV; ++v) acc[v] = 0.0;
-  // one term D_split(x_d, m) f(u_a, u_b) of line direction d, partner m
-  auto term = [&](int d, int xd, int sd, int m, const double* jown) {
-    const int pb = lds_pos<N>(a + (m - xd) * sd);
-    NodePrims<DIM> qb;
-    qb.rho = s_q[pb];
+  // One term D_split(x_d, m) f(u_a, u_b) of line direction d, partner m at LDS
+  // position pb.  The node's own metric row is read again from LDS for each
+  // term (affine: the element's, from the registers): selecting it from
+  // registers by the lane's direction costs more than the three reads.
+  auto term = [&](int d, int xd, int m, int pb) {
+    PairNode<DIM> qb;
+    qb.r = s_q[pb];
 #pragma unroll
     for (int c = 0; c < DIM; ++c) qb.v[c] = s_q[(1 + c) * PN + pb];
-    qb.beta = s_q[QB * PN + pb];
+    qb.b = s_q[QB * PN + pb];
     qb.kin = s_q[(QB + 1) * PN + pb];
-    qb.p = 0.0;
-    qb.c = 0.0;
     double nrm[DIM], f[NV];
+    if constexpr (NODAL) {
+      // (Ja_x + Ja_m) / 2 from the halved rows (halving is exact)
+      const double* row = s_ja + d * (DIM * PN);
 #pragma unroll
-    for (int c = 0; c < DIM; ++c) {
-      // NODAL: (Ja_x + Ja_m) / 2 from the halved rows (halving is exact)
-      nrm[c] = NODAL ? jown[c] + s_ja[(d * DIM + c) * PN + pb] : jown[c];
+      for (int c = 0; c < DIM; ++c) nrm[c] = row[c * PN + pa] + row[c * PN + pb];
+    } else {
+#pragma unroll
+      for (int c = 0; c < DIM; ++c) {
+        nrm[c] = d == 0 ? jm[0][c] : jm[1][c];
+        if constexpr (DIM == 3) nrm[c] = d == 2 ? jm[2][c] : nrm[c];
+      }
     }
-    flux_chandrashekar_exact<DIM>(p.inv_gm1, q, qb, nrm, f);
+    flux_chandrashekar_exact<DIM>(p.inv_gm1, qa, qb, nrm, f);
     const double w = s_D[xd * DS + m];
 #pragma unroll
     for (int v = 0; v < NV; ++v) {
 #pragma clang fp contract(off)
-      acc[v] = acc[v] + w * f[v];
+      acc[v] = acc[v] + (v == NV - 1 ? 0.5 * w : w) * f[v];
     }
   };
-  // the node's own rows (NODAL: halved, from LDS; affine: the element's)
-  double jx[DIM], jy[DIM], jz[DIM];
-#pragma unroll
-  for (int c = 0; c < DIM; ++c) {
-    jx[c] = NODAL ? s_ja[(0 * DIM + c) * PN + pa] : jm[0][c];
-    jy[c] = NODAL ? s_ja[(1 * DIM + c) * PN + pa] : jm[1][c];
-    jz[c] = DIM == 3 ? (NODAL ? s_ja[((DIM - 1) * DIM + c) * PN + pa] : jm[DIM - 1][c]) : 0.0;
-  }
+  // LDS positions of the node's lines' first nodes and their strides
+  constexpr int PY = n + 1, PZ = n * (n + 1);
+  const int xb = pa - ix, yb = pa - iy * PY, zb = DIM == 3 ? pa - iz * PZ : 0;
+  // The lane's term t of its y- and x-lines: below on the y-line, below and
+  // above on the x-line, above on the y-line (2N terms for every node).
+  auto xy_term = [&](int t, bool& dy, int& m) {
+    dy = t < iy || t >= iy + N;
+    m = dy ? (t < iy ? t : t + 1 - N) : (t < iy + ix ? t - iy : t - iy + 1);
+  };
   // partners below on the z-line (3D)
   if constexpr (DIM == 3) {
 #pragma unroll 1
-    for (int m = 0; m < iz; ++m) term(2, iz, n * n, m, jz);
+    for (int m = 0; m < iz; ++m) term(2, iz, m, zb + m * PZ);
   }
-  // below on the y-line, below and above on the x-line, above on the y-line:
-  // 2N terms for every node
 #pragma unroll 1
   for (int t = 0; t < 2 * N; ++t) {
-    const bool yl = t < iy, xl = t < iy + ix, xu = t < iy + N;
-    const bool dy = yl || !xu;
-    const int m = yl ? t : (xl ? t - iy : (xu ? t - iy + 1 : t - N + 1));
-    double jo[DIM];
-#pragma unroll
-    for (int c = 0; c < DIM; ++c) jo[c] = dy ? jy[c] : jx[c];
-    term(dy ? 1 : 0, dy ? iy : ix, dy ? n : 1, m, jo);
+    bool dy;
+    int m;
+    xy_term(t, dy, m);
+    term(dy ? 1 : 0, dy ? iy : ix, m, dy ? yb + m * PY : xb + m);
   }
   // partners above on the z-line (3D)
   if constexpr (DIM == 3) {
 #pragma unroll 1
-    for (int m = iz + 1; m <= N; ++m) term(2, iz, n * n, m, jz);
+    for (int m = iz + 1; m <= N; ++m) term(2, iz, m, zb + m * PZ);
   }
+
+  // 4. numerical fluxes on the element's faces, one thread for each line end:
+  // thread (dir, side, line) of the first FACE threads, so that a wave takes
+  // one side of one direction (3D) and every lane works.  Formed by the face
+  // nodes' own threads they ran once per direction in every wave, a quarter of
+  // its lanes active.  The lower face takes the lower neighbour's node with
+  // index N, the upper face the upper neighbour's node with index 0 and its
+  // metric row and 1/J, whose sign and row make the interface normal.
+  {
+    const bool has_face = a < FACE;
+    const int fd = a / (2 * FN), rem = a - fd * (2 * FN), line = rem % FN;
+    const bool lower = rem < FN;
+    double f[NV];
+    if (has_face) {
+      const LineNodes<DIM, N> ln(fd, line);
+      const int first = ln.base, last = ln.base + N * ln.stride;
+      int64_t lo, hi;
+      face_neighbours<DIM, false>(p, eid, e, fd, lo, hi);
+      const int64_t ne = lower ? lo : hi;
+      const int on = lower ? first : last, nn = lower ? last : first;
+      const double* uo = p.u + e * (NV * NN) + on;
+      const double* un = p.u + ne * (NV * NN) + nn;
+      // the face's upper element, whose first node makes the normal
+      const int64_t ue = lower ? e : hi;
+      const double uij = NODAL ? p.invJ[ue * NN + first] : p.invJ[ue];
+      const double sg = uij >= 0.0 ? 1.0 : -1.0;
+      double so[NV], sn[NV], ul[NV], ur[NV], nrm[DIM];
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        so[v] = uo[v * NN];
+        sn[v] = un[v * NN];
+      }
+#pragma unroll
+      for (int c = 0; c < DIM; ++c)
+        nrm[c] = sg * (NODAL ? p.Ja[((ue * DIM + fd) * DIM + c) * NN + first]
+                             : p.Ja[(ue * DIM + fd) * DIM + c]);
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        ul[v] = lower ? sn[v] : so[v];
+        ur[v] = lower ? so[v] : sn[v];
+      }
+      if constexpr (SF == kFluxLLF) {
+        flux_llf_exact<DIM>(p.gamma, ul, ur, nrm, f);
+      } else {
+        flux_hllc_exact<DIM>(p.gamma, ul, ur, nrm, f);
+      }
+    }
+    __syncthreads();  // the term loops are done with the primitives
+    if (has_face) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) s_face[((fd * 2 + (lower ? 0 : 1)) * NV + v) * FN + line] = f[v];
+    }
+  }
+
   // 3b. Navier-Stokes: the viscous volume integral adds
   // D_hat(x_d, m) Ja^d . (-F_v)(m) over every partner m of each line through
   // the node (the node itself included) into the same sums, after the
@@ -391,43 +487,60 @@ __global__ void __launch_bounds__((Shape<DIM, N>::NN)) __attribute__((amdgpu_wav
   // terms, then the rest of its x-, y- and z-lines.  At a face node the sums
   // hold the uncancelled half of the face balance, about a thousand times
   // the RHS, so this order fixes the RHS's last bits whatever the viscosity.
+  // The element's fluxes are staged in the planes the term loops have left;
+  // the mass component is zero and adds nothing.
   const double* vf = p.visc;  // [E][d][var][dof], or null (Euler)
-  auto vterm = [&](int d, int xd, int sd, int m) {
-    const int b = a + (m - xd) * sd;
-    const double w = s_Dh[xd * DS + m];
+  if (vf) {
+    double own[DIM][NV - 1];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) {
-#pragma clang fp contract(off)
-      acc[v] = acc[v] + w * vf[((e * DIM + d) * NV + v) * NN + b];
-    }
-  };
-  if (vf) {
-    if constexpr (DIM == 3) {
-#pragma unroll 1
-      for (int m = 0; m < iz; ++m) vterm(2, iz, n * n, m);
-    }
-#pragma unroll 1
-    for (int m = 0; m < iy; ++m) vterm(1, iy, n, m);
-#pragma unroll 1
-    for (int m = 0; m <= ix; ++m) vterm(0, ix, 1, m);
-    vterm(1, iy, n, iy);
-    if constexpr (DIM == 3) vterm(2, iz, n * n, iz);
-#pragma unroll 1
-    for (int m = ix + 1; m <= N; ++m) vterm(0, ix, 1, m);
-#pragma unroll 1
-    for (int m = iy + 1; m <= N; ++m) vterm(1, iy, n, m);
-    if constexpr (DIM == 3) {
-#pragma unroll 1
-      for (int m = iz + 1; m <= N; ++m) vterm(2, iz, n * n, m);
-    }
+    for (int d = 0; d < DIM; ++d)
+#pragma unroll
+      for (int v = 1; v < NV; ++v) own[d][v - 1] = vf[((e * DIM + d) * NV + v) * NN + a];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d)
+#pragma unroll
+      for (int v = 1; v < NV; ++v) s_vf[(d * (NV - 1) + v - 1) * PN + pa] = own[d][v - 1];
   }
-  const double own_sg = ij >= 0.0 ? 1.0 : -1.0;
-  // 3c. the viscous interface terms in direction order
-  // (structured_solver.hpp:359-360 with the one-sided flux of
-  // parabolic_viscous.hpp:318-334 / :570-585): the lower face takes the
-  // node's own (-F_v) . (sign(J) Ja^d), the upper face the upper
-  // neighbour's at its node with index 0.
+  __syncthreads();
   if (vf) {
+    auto vterm = [&](int d, int xd, int m, int pb) {
+      const double w = s_Dh[xd * DS + m];
+      const double* g = s_vf + d * ((NV - 1) * PN) + pb;
+#pragma unroll
+      for (int v = 1; v < NV; ++v) {
+#pragma clang fp contract(off)
+        acc[v] = acc[v] + w * g[(v - 1) * PN];
+      }
+    };
+    if constexpr (DIM == 3) {
+#pragma unroll 1
+      for (int m = 0; m < iz; ++m) vterm(2, iz, m, zb + m * PZ);
+    }
+    // y below, x up to the node, the node's own y and z, the rest of x and y:
+    // the same terms as xy_term with the node itself among them
+#pragma unroll 1
+    for (int t = 0; t <= iy + ix; ++t) {
+      const bool dy = t < iy;
+      const int m = dy ? t : t - iy;
+      vterm(dy ? 1 : 0, dy ? iy : ix, m, dy ? yb + m * PY : xb + m);
+    }
+    vterm(1, iy, iy, pa);
+    if constexpr (DIM == 3) vterm(2, iz, iz, pa);
+#pragma unroll 1
+    for (int t = 0; t < 2 * N - ix - iy; ++t) {
+      const bool dy = t >= N - ix;
+      const int m = dy ? iy + 1 + t - (N - ix) : ix + 1 + t;
+      vterm(dy ? 1 : 0, dy ? iy : ix, m, dy ? yb + m * PY : xb + m);
+    }
+    if constexpr (DIM == 3) {
+#pragma unroll 1
+      for (int m = iz + 1; m <= N; ++m) vterm(2, iz, m, zb + m * PZ);
+    }
+    // 3c. the viscous interface terms in direction order
+    // (structured_solver.hpp:359-360 with the one-sided flux of
+    // parabolic_viscous.hpp:318-334 / :570-585): the lower face takes the
+    // node's own (-F_v) . (sign(J) Ja^d), the upper face the upper
+    // neighbour's at its node with index 0.
 #pragma unroll
     for (int d = 0; d < DIM; ++d) {
       const bool lower = idx[d] == 0, upper = idx[d] == N;
@@ -439,7 +552,7 @@ __global__ void __launch_bounds__((Shape<DIM, N>::NN)) __attribute__((amdgpu_wav
         const double vij = lower ? ij : (NODAL ? p.invJ[ve * NN + vn] : p.invJ[ve]);
         const double sg = vij >= 0.0 ? 1.0 : -1.0;
 #pragma unroll
-        for (int v = 0; v < NV; ++v) {
+        for (int v = 1; v < NV; ++v) {
 #pragma clang fp contract(off)
           const double fp = sg * vf[((ve * DIM + d) * NV + v) * NN + vn];
           acc[v] = lower ? acc[v] - fp * p.lhat0 : acc[v] + fp * p.lhatN;
@@ -447,50 +560,19 @@ __global__ void __launch_bounds__((Shape<DIM, N>::NN)) __attribute__((amdgpu_wav
       }
     }
   }
-  // 4. numerical fluxes on the faces this node lies on, lifted after the
-  // volume terms in direction order.  Their inputs are loaded here, not at
-  // the top, so that nothing but the sums lives through the term loops (a
-  // value held across them would spill).  The lower face takes the lower
-  // neighbour's node with index N, the upper face the upper neighbour's node
-  // with index 0 and its metric row and 1/J, whose sign and row make the
-  // interface normal; interior nodes load nothing.
+  // 4b. the face fluxes, lifted in direction order
 #pragma unroll
   for (int d = 0; d < DIM; ++d) {
     const bool lower = idx[d] == 0, upper = idx[d] == N;
     if (lower || upper) {
-      int64_t lo, hi;
-      face_neighbours<DIM, false>(p, eid, e, d, lo, hi);
-      const int64_t ne = lower ? lo : hi;
-      const int nn = lower ? a + N * stride[d] : a - N * stride[d];
-      double un[NV], uo[NV], nrm[DIM], f[NV];
-#pragma unroll
-      for (int v = 0; v < NV; ++v) {
-        un[v] = p.u[(ne * NV + v) * NN + nn];
-        uo[v] = p.u[(e * NV + v) * NN + a];
-      }
-      if (lower) {
-#pragma unroll
-        for (int c = 0; c < DIM; ++c)
-          nrm[c] = own_sg * (NODAL ? 2.0 * s_ja[(d * DIM + c) * PN + pa] : jm[d][c]);
-      } else {
-        const double nij = NODAL ? p.invJ[ne * NN + nn] : p.invJ[ne];
-        const double nb_sg = nij >= 0.0 ? 1.0 : -1.0;
-#pragma unroll
-        for (int c = 0; c < DIM; ++c)
-          nrm[c] = nb_sg * (NODAL ? p.Ja[((ne * DIM + d) * DIM + c) * NN + nn]
-                                  : p.Ja[(ne * DIM + d) * DIM + c]);
-      }
-      const double* ul = lower ? un : uo;
-      const double* ur = lower ? uo : un;
-      if constexpr (SF == kFluxLLF) {
-        flux_llf_exact<DIM>(p.gamma, ul, ur, nrm, f);
-      } else {
-        flux_hllc_exact<DIM>(p.gamma, ul, ur, nrm, f);
-      }
+      // line of the node in direction d
+      const int line = DIM == 2 ? idx[1 - d]
+                                : idx[d == 2 ? 1 : 2] * n + idx[d == 0 ? 1 : 0];
+      const double* f = s_face + (d * 2 + (lower ? 0 : 1)) * (NV * FN) + line;
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
 #pragma clang fp contract(off)
-        acc[v] = lower ? acc[v] - f[v] * p.lhat0 : acc[v] + f[v] * p.lhatN;
+        acc[v] = lower ? acc[v] - f[v * FN] * p.lhat0 : acc[v] + f[v * FN] * p.lhatN;
       }
     }
   }

@@ -332,7 +332,7 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) viscous_kernel(c
 // Ja^d_0 f_0 + Ja^d_1 f_1 (+ Ja^d_2 f_2) from left to right, with no fused
 // multiply-adds.  The interface value (-F_v) . (sign(J) Ja^d) of a face node
 // is sign(J) times this sum to the bit (scaling by a sign is exact), so the
-// RHS kernel needs nothing more.
+// RHS kernel needs nothing more.  The mass component is zero: not stored.
 template <int DIM, int N, bool NODAL>
 __device__ __forceinline__ void store_viscous_fluxes(const KParams& p, int64_t e, int node,
                                                      const double* q, const double g[DIM][DIM + 2]) {
@@ -346,7 +346,7 @@ __device__ __forceinline__ void store_viscous_fluxes(const KParams& p, int64_t e
 #pragma unroll
     for (int c = 0; c < DIM; ++c) ja[c] = metric<NODAL, DIM, NN>(p, e, d, c, node);
 #pragma unroll
-    for (int v = 0; v < NV; ++v) {
+    for (int v = 1; v < NV; ++v) {
 #pragma clang fp contract(off)
       double r = ja[0] * -fv[0][v];
 #pragma unroll
