@@ -218,13 +218,6 @@ bool has_boundaries(const dgsem_config& c) {
   return false;
 }
 
-// Navier-Stokes viscous buffer: the node-parallel RHS kernel takes the
-// per-node fluxes of every direction, the line kernels the viscous RHS part.
-int64_t visc_width(const dgsem_config& c) {
-  const bool sc = c.volume_integral == DGSEM_VOLUME_SHOCK_CAPTURING;
-  return dgsem::node_kernel_for(c.polydeg, sc, has_boundaries(c)) ? c.dim : 1;
-}
-
 int check_config(dgsem_handle* h, const dgsem_config& c) {
   if (c.dim != 2 && c.dim != 3) return fail(h, DGSEM_E_INVALID, "dim must be 2 or 3");
   if (c.polydeg < 1 || c.polydeg > 7) return fail(h, DGSEM_E_INVALID, "polydeg must be 1..7");
@@ -284,8 +277,8 @@ int launch(dgsem_handle* h, dgsem::KParams p) {
   const bool sc = h->cfg.volume_integral == DGSEM_VOLUME_SHOCK_CAPTURING;
   const bool nodal = h->cfg.geometry == DGSEM_GEOMETRY_NODAL;
   if (h->cfg.equation == DGSEM_NAVIER_STOKES) {
-    // BR1 gradient and viscous part of the stage input, then the inviscid
-    // kernel adds the viscous part before -1/J
+    // viscous fluxes of the stage input, then the inviscid kernel adds their
+    // divergence and interface terms before -1/J
     hipError_t e = dgsem::launch_parabolic(h->cfg.dim, h->cfg.polydeg, sc, nodal, has_boundaries(h->cfg),
                                            p, stream_of(h));
     if (e != hipSuccess) return hip_fail(h, e, "parabolic kernel launch");
@@ -409,17 +402,17 @@ int dgsem_create(const dgsem_config* cfg, void* stream, dgsem_handle** out) {
   std::vector<double> sn;
   if (h->cfg.geometry == DGSEM_GEOMETRY_NODAL && h->cfg.volume_integral == DGSEM_VOLUME_SHOCK_CAPTURING)
     sn = h->geo.subcell_normals;
+  const bool node_kernel = dgsem::node_kernel_for(
+      h->cfg.polydeg, h->cfg.volume_integral == DGSEM_VOLUME_SHOCK_CAPTURING, has_boundaries(h->cfg));
   if ((rc = upload(h, &h->d_Ja, Ja)) || (rc = upload(h, &h->d_invJ, invJ)) ||
       (rc = upload(h, &h->d_sn, sn)) || (rc = upload(h, &h->d_nbr, neighbour_table(h->geo, periodic))) ||
       (rc = upload(h, &h->d_Vinv, h->basis.Vinv)) ||
       (rc = upload(h, &h->d_alpha, std::vector<double>(4 * h->E, 0.0))) ||
-      // Navier-Stokes: the per-node gradient only where the line kernels
-      // read it (the node-parallel path keeps the viscous fluxes alone; the
-      // tangent and adjoint allocate the gradient when they first need it)
+      // Navier-Stokes: the viscous fluxes, and the gradient of the tangent and
+      // adjoint (which allocate it themselves where the node kernel runs)
       (h->cfg.equation == DGSEM_NAVIER_STOKES &&
-       ((visc_width(h->cfg) == 1 &&
-         (rc = alloc_zero(h, &h->d_grad, (size_t)h->E * h->cfg.dim * h->nvars * h->nn))) ||
-        (rc = alloc_zero(h, &h->d_visc, (size_t)h->E * visc_width(h->cfg) * h->nvars * h->nn))))) {
+       ((!node_kernel && (rc = alloc_zero(h, &h->d_grad, (size_t)h->E * h->cfg.dim * h->nvars * h->nn))) ||
+        (rc = alloc_zero(h, &h->d_visc, (size_t)h->E * h->cfg.dim * h->nvars * h->nn))))) {
     release(h);
     *out = h;
     return rc;

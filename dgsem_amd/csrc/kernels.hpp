@@ -15,9 +15,7 @@ constexpr int kMaxN1 = 8;  // max nodes per direction (N <= 7)
 #endif
 
 // Split-form elements of degree N >= 7 on periodic meshes run the
-// node-parallel kernel, in 2D and 3D.  With Navier-Stokes terms that kernel
-// takes the viscous fluxes Ja^d . (-F_v) per node [E][dim][var][dof]
-// (instead of their divergence [E][var][dof]) and adds their terms itself.
+// node-parallel kernel, in 2D and 3D.
 __host__ __device__ constexpr bool node_kernel_for(int N, bool shock_capturing, bool boundaries) {
   return !shock_capturing && !boundaries && N >= DGSEM_NODE_KERNEL_MIN_N;
 }
@@ -81,7 +79,7 @@ struct KParams {
   const double* Vinv;    // [n][n] inverse Legendre Vandermonde
   const double* grad;    // Navier-Stokes: gradient [E][dim][var][dof]
   double* grad_out;      // written by the gradient kernel
-  const double* visc;    // Navier-Stokes: viscous part of the RHS before -1/J
+  const double* visc;    // Navier-Stokes: viscous fluxes (parabolic_impl.hpp)
   double* visc_out;      // written by the viscous kernel
   int64_t E;
   int mode;
@@ -115,10 +113,8 @@ template <int DIM, int N>
 hipError_t launch_parabolic_dn(bool shock_capturing, bool nodal, bool boundaries, const KParams& p,
                                hipStream_t stream);
 
-// Gradient and viscous kernels of the Navier-Stokes terms: fill p.grad_out
-// (with p.grad == p.grad_out) and p.visc_out from p.u; p.visc_out takes the
-// per-node viscous fluxes when node_kernel_for(N, shock_capturing,
-// boundaries), else the viscous part of the RHS.
+// The Navier-Stokes terms: the viscous fluxes of p.u into p.visc_out, in the
+// layout the RHS kernel of the configuration reads (parabolic_impl.hpp).
 hipError_t launch_parabolic(int dim, int N, bool shock_capturing, bool nodal, bool boundaries,
                             const KParams& p, hipStream_t stream);
 

@@ -1,27 +1,28 @@
 // BR1 parabolic terms of the compressible Navier-Stokes RHS on the GPU.
 //
-// Two kernels per RHS, both one workgroup per EPW elements with line threads
-// as in the inviscid kernel:
-//   * gradient_kernel: q = (rho, v, T) at the nodes; along each line the weak
-//     derivative D_hat q, the BR1 face value q_hat = (q_L + q_R)/2 lifted
-//     with l_hat; then the physical gradient sum_d Ja^d (.) and 1/J.
-//     Reference: GradientVolumeIntegralFunctor, GradientPhysicalTransform-
-//     Functor, GradientInterfaceFluxFunctor, GradientSurfaceIntegralFunctor,
-//     GradientJacobianProjFunctor (parabolic_gradient.hpp:17-478 3D,
-//     :480-818 2D).
-//   * viscous_kernel: the contravariant viscous flux Ja^d . (-F_v) at the
-//     nodes, its weak D_hat divergence along each line, and the interface
-//     flux, which is the upper ("primary") element's (-F_v).n only
-//     (parabolic_viscous.hpp:318-334 3D, :570-585 2D), lifted with l_hat.
-//     The result (before -1/J) is added by the inviscid kernel.
-//     Elements of the node-parallel RHS kernel (node_kernel_for) take
-//     gradient_node_kernel instead, which stores the per-node viscous fluxes
-//     only; that kernel adds their terms in the reference's order.
-// Layouts: gradient [E][dim][var][dof]; viscous part [E][var][dof], or the
-// per-node fluxes [E][dim][var][dof].
+// One kernel before the inviscid one forms the contravariant viscous flux
+// Ja^d . (-F_v) at every node: q = (rho, v, T); along each line the weak
+// derivative D_hat q, the BR1 face value q_hat = (q_L + q_R)/2 lifted with
+// l_hat; the physical gradient sum_d Ja^d (.) / J; the flux.  The gradient
+// itself never goes to memory, nor does anything of rho, which the viscous
+// flux does not differentiate, nor the flux's zero mass component.  Reference:
+// GradientVolumeIntegralFunctor, GradientPhysicalTransformFunctor,
+// GradientInterfaceFluxFunctor, GradientSurfaceIntegralFunctor,
+// GradientJacobianProjFunctor (parabolic_gradient.hpp:17-478 3D, :480-818 2D)
+// and ViscousFluxFunctor (parabolic_viscous.hpp:39-66 3D, :367-386 2D).
+//   * viscous_flux_kernel: line threads, for the line kernels (rhs_kernel),
+//     whose line threads form the flux's D_hat divergence and the interface
+//     flux, the upper ("primary") element's (-F_v).n only
+//     (parabolic_viscous.hpp:318-334 3D, :570-585 2D), beside the pair fluxes.
+//     Layout [E][d][var][line * n + k]: node k of line `line` of direction d,
+//     so that a line thread reads contiguous runs.
+//   * gradient_node_kernel: for the elements of the node-parallel RHS kernel
+//     (node_kernel_for), rounded as the reference; layout [E][d][var][dof].
+// gradient_kernel writes the gradient [E][dim][var][dof] for the tangent and
+// adjoint kernels.
 // BCS (2D): some face is not periodic; the neighbour table holds -1 there and
 // the face values come from the boundary condition (wall_gradient_value and
-// the viscous kernel's wall branch).
+// rhs_kernel's wall branch).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -189,138 +190,197 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) gradient_kernel(
   }
 }
 
-// Contravariant viscous flux Ja^d . (-F_v) of one node: out[d][v].
-template <int DIM, int NN, bool NODAL>
-__device__ __forceinline__ void contravariant_viscous(const KParams& p, int64_t e, int node,
-                                                      const double* u, double out[DIM][DIM + 2]) {
-  constexpr int NV = DIM + 2;
-  double q[NV], g[DIM][NV], fv[DIM][NV];
-  grad_vars<DIM>(p.gamma, u, q);
-  for (int c = 0; c < DIM; ++c)
-    for (int v = 0; v < NV; ++v) g[c][v] = p.grad[((e * DIM + c) * NV + v) * NN + node];
-  for (int c = 0; c < DIM; ++c) viscous_flux_dir<DIM>(p.mu, p.kappa, q, g, c, fv[c]);
-  for (int d = 0; d < DIM; ++d) {
-    double ja[DIM];
-    for (int c = 0; c < DIM; ++c) ja[c] = metric<NODAL, DIM, NN>(p, e, d, c, node);
-    for (int v = 0; v < NV; ++v) {
-      double r = 0.0;
-      for (int c = 0; c < DIM; ++c) r += ja[c] * -fv[c][v];
-      out[d][v] = r;
-    }
-  }
+// Position of node `dof` in the direction-d rows line * n + k (LineNodes).
+template <int DIM, int N>
+__device__ __forceinline__ int row_pos(int d, int dof) {
+  constexpr int n = N + 1;
+  if (d == 0) return dof;
+  const int ix = dof % n, iy = (dof / n) % n, iz = dof / (n * n);
+  if constexpr (DIM == 2) return ix * n + iy;
+  return d == 1 ? (iz * n + ix) * n + iy : (iy * n + ix) * n + iz;
 }
 
-template <int DIM, int N, int EPW, bool NODAL, bool BCS>
-__global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) viscous_kernel(const KParams p) {
-  using S = Shape<DIM, N>;
-  constexpr int n = S::n, NV = S::NV, NN = S::NN, FN = S::FN, L = S::LINES;
-  constexpr int BLOCK = EPW * L;
-  __shared__ double s_f[EPW * DIM * NV * NN];  // Ja^d . (-F_v) per node and d
-  __shared__ double s_du[EPW * NV * NN];
-  const int tid = threadIdx.x;
-  const int blk = xcd_block(blockIdx.x, gridDim.x);
-  const int64_t e0 = (int64_t)blk * EPW;
-  const int nvalid = (int)((p.E - e0) < EPW ? (p.E - e0) : EPW);
+// Metric terms Ja^d_c of a node, from the box table (rows of halved terms) or
+// the per-node arrays.
+template <int DIM, int N, bool NODAL, bool BOX>
+__device__ __forceinline__ void node_metric(const KParams& p, int64_t e, const int* eid, int dof,
+                                            double ja[DIM][DIM]) {
+  constexpr int NN = Shape<DIM, N>::NN;
+#pragma unroll
+  for (int d = 0; d < DIM; ++d)
+#pragma unroll
+    for (int c = 0; c < DIM; ++c)
+      ja[d][c] = BOX ? 2.0 * box_row<DIM, N>(p, eid, c, d, 0)[row_pos<DIM, N>(d, dof)]
+                     : metric<NODAL, DIM, NN>(p, e, d, c, dof);
+}
 
-  for (int i = tid; i < EPW * NN; i += BLOCK) {
-    const int sl = i / NN, node = i % NN;
-    if (sl >= nvalid) continue;
-    const int64_t e = e0 + sl;
-    double s[NV], out[DIM][NV];
-    for (int v = 0; v < NV; ++v) s[v] = p.u[(e * NV + v) * NN + node];
-    contravariant_viscous<DIM, NN, NODAL>(p, e, node, s, out);
-    for (int d = 0; d < DIM; ++d)
-      for (int v = 0; v < NV; ++v) s_f[((sl * DIM + d) * NV + v) * NN + node] = out[d][v];
+// The nodes' viscous fluxes into p.visc_out (see the top of the file).  Memory
+// bound: a node reads its state (and, off a box mesh, its metric terms) and
+// writes DIM (DIM + 1) fluxes.  Whole-node staging, line threads and LDS planes
+// as in rhs_kernel; the line derivatives take the place of q in LDS, so that
+// five blocks of the 3D N = 3 kernel fit a CU.  Storing the fluxes instead of
+// the gradient, with the divergence in rhs_kernel, replaced a gradient and a
+// viscous-divergence kernel (85 -> 46 doubles of traffic per node and stage on a
+// box mesh): SSPRK3 step at 32^3 N = 3 1.10 -> 0.57 ms, 2D shock tube 200 x 100
+// N = 3 with walls, 12 stages, 468 -> 316 us.
+template <int DIM, int N, int EPW, bool NODAL, bool BCS, bool BOX>
+__global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) viscous_flux_kernel(const KParams p) {
+  using S = Shape<DIM, N>;
+  constexpr int n = S::n, NV = S::NV, NN = S::NN, FN = S::FN, PN = S::PN;
+  constexpr int ND = NV - 1;  // differentiated variables v, T: planes v - 1
+  constexpr int BLOCK = EPW * S::LINES, NODES = EPW * NN, PASSES = (NODES + BLOCK - 1) / BLOCK;
+  constexpr int SG = DIM * ND * PN + S::slot_pad(DIM * ND * PN);
+  __shared__ double s_g[EPW * SG];  // q [var], later D_hat q + lift [dir][var]
+  const int tid = threadIdx.x;
+  const int64_t e0 = (int64_t)xcd_block(blockIdx.x, gridDim.x) * EPW;
+  const int nvalid = (int)((p.E - e0) < EPW ? (p.E - e0) : EPW);
+  auto has_node = [&](int k) { return (k + 1) * BLOCK <= NODES || tid + k * BLOCK < NODES; };
+
+  // node states; slots past the last valid element take a copy of it
+  double q[PASSES][NV];
+#pragma unroll
+  for (int k = 0; k < PASSES; ++k) {
+    if (has_node(k)) {
+      const int i = tid + k * BLOCK, sl = i / NN, node = i - sl * NN;
+      const double* src = p.u + (e0 + (sl < nvalid ? sl : nvalid - 1)) * (NV * NN) + node;
+#pragma unroll
+      for (int v = 0; v < NV; ++v) q[k][v] = src[v * NN];
+    }
+  }
+  // the line and its neighbours' traces, threads ordered (dir, slot, line)
+  const int dir = tid / (EPW * FN), rem = tid % (EPW * FN), slot = rem / FN, line = rem % FN;
+  const bool valid = slot < nvalid && dir < DIM;
+  const int64_t el = valid ? e0 + slot : e0;
+  const int dl = dir < DIM ? dir : DIM - 1;
+  const LineNodes<DIM, N> ln(dl, line);
+  const int first = ln.base, last = ln.base + N * ln.stride;
+  int eid[3];
+  element_indices<DIM>(p, (int)el, eid);
+  int64_t nb_lo, nb_hi;
+  face_neighbours<DIM, BCS>(p, eid, el, dl, nb_lo, nb_hi);
+  const bool blo = BCS && nb_lo < 0, bhi = BCS && nb_hi < 0;
+  double t_lo[NV], t_hi[NV];
+  {
+    const double* ulo = p.u + (blo ? el : nb_lo) * (NV * NN) + last;
+    const double* uhi = p.u + (bhi ? el : nb_hi) * (NV * NN) + first;
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      t_lo[v] = ulo[v * NN];
+      t_hi[v] = uhi[v * NN];
+    }
+  }
+  // the face terms use the element's own normal sign(J) Ja^dir at its nodes
+  const double sg_lo = BOX || inv_jac<NODAL, NN>(p, el, first) >= 0.0 ? 1.0 : -1.0;
+  const double sg_hi = BOX || inv_jac<NODAL, NN>(p, el, last) >= 0.0 ? 1.0 : -1.0;
+#pragma unroll
+  for (int k = 0; k < PASSES; ++k) {
+    if (has_node(k)) {
+      const int i = tid + k * BLOCK, sl = i / NN, pn = lds_pos<N>(i - sl * NN);
+      double u[NV];
+#pragma unroll
+      for (int v = 0; v < NV; ++v) u[v] = q[k][v];
+      grad_vars<DIM>(p.gamma, u, q[k]);
+#pragma unroll
+      for (int v = 1; v < NV; ++v) s_g[sl * SG + (v - 1) * PN + pn] = q[k][v];
+    }
   }
   __syncthreads();
-
-  const int slot = tid / L, rem = tid % L, dir = rem / FN, line = rem % FN;
-  const bool valid = slot < nvalid;
-  double acc[n][NV];
-  int dofs[n];
-#pragma unroll
-  for (int k = 0; k < n; ++k) dofs[k] = line_dof<DIM, N>(dir, line, k);
-  if (valid) {
-    const int64_t e = e0 + slot;
-    const double* f = s_f + (slot * DIM + dir) * NV * NN;
+  double acc[n][ND];
+  {
+    double x[n][ND];
 #pragma unroll
     for (int k = 0; k < n; ++k)
 #pragma unroll
-      for (int v = 0; v < NV; ++v) {
+      for (int v = 0; v < ND; ++v) x[k][v] = s_g[slot * SG + v * PN + ln.pbase + k * ln.pstride];
+#pragma unroll
+    for (int k = 0; k < n; ++k)
+#pragma unroll
+      for (int v = 0; v < ND; ++v) {
         double r = 0.0;
 #pragma unroll
-        for (int i = 0; i < n; ++i) r += p.Dhat[k][i] * f[v * NN + dofs[i]];
+        for (int i = 0; i < n; ++i) r += p.Dhat[k][i] * x[i][v];
         acc[k][v] = r;
       }
-    // Boundary faces (BCS): the own node's (-F_v).(sign(J) Ja^dir) for the
-    // momentum components only at a no-slip adiabatic wall
-    // (navier_stokes_wall_boundary.hpp:116-145), for every variable at a
-    // Dirichlet face (dirichlet_boundary.hpp:164-194); every other kind
-    // leaves the face value at zero (:199-216, boundary_set.hpp:35-51).
-    bool bnd_lo = false, bnd_hi = false;
-    int vlo[2] = {0, 0}, vhi[2] = {0, 0};  // variables carried, per side
+    // BR1 face values q_hat = (q_lower + q_upper) / 2 on both line ends
+    double q_lo[NV], q_hi[NV];
+    grad_vars<DIM>(p.gamma, t_lo, q_lo);
+    grad_vars<DIM>(p.gamma, t_hi, q_hi);
+#pragma unroll
+    for (int v = 1; v < NV; ++v) {
+      q_lo[v] = 0.5 * (q_lo[v] + x[0][v - 1]);
+      q_hi[v] = 0.5 * (x[n - 1][v - 1] + q_hi[v]);
+    }
     if constexpr (BCS) {
-      bnd_lo = p.nbr[e * 2 * DIM + 2 * dir] < 0;
-      bnd_hi = p.nbr[e * 2 * DIM + 2 * dir + 1] < 0;
-      for (int side = 0; side < 2; ++side) {
-        const int kind = p.bc[2 * dir + side];
-        vlo[side] = kind == kBcDirichlet ? 0 : 1;
-        vhi[side] = kind == kBcDirichlet ? NV : (kind == kBcNsNoSlipWall ? NV - 1 : 0);
+      auto wall = [&](int side, int dof, double sg, const double* xn, double* out) {
+        const int face = 2 * dl + side;
+        if (p.bc[face] == kBcDirichlet) {
+          const int64_t bnode = (int64_t)(dl == 0 ? eid[1] : eid[0]) * n + line;
+          const double* vals = p.bc_values[face];
+          double so[NV];
+          for (int v = 0; v < NV; ++v) so[v] = vals ? vals[bnode * NV + v] : p.bc_state[face][v];
+          grad_vars<DIM>(p.gamma, so, out);
+        } else {
+          double own[NV], nrm[DIM];
+          own[0] = 0.0;  // rho: not differentiated
+          for (int v = 1; v < NV; ++v) own[v] = xn[v - 1];
+          for (int c = 0; c < DIM; ++c) nrm[c] = sg * metric<NODAL, DIM, NN>(p, el, dl, c, dof);
+          wall_gradient_value<DIM>(p.bc[face], own, nrm, out);
+        }
+      };
+      if (blo) wall(0, first, sg_lo, x[0], q_lo);
+      if (bhi) wall(1, last, sg_hi, x[n - 1], q_hi);
+    }
+#pragma unroll
+    for (int v = 1; v < NV; ++v) {
+      acc[0][v - 1] -= sg_lo * p.lhat0 * q_lo[v];
+      acc[n - 1][v - 1] += sg_hi * p.lhatN * q_hi[v];
+    }
+  }
+  __syncthreads();  // every line has read its q
+  if (dir < DIM) {
+#pragma unroll
+    for (int k = 0; k < n; ++k)
+#pragma unroll
+      for (int v = 0; v < ND; ++v)
+        s_g[slot * SG + (dir * ND + v) * PN + ln.pbase + k * ln.pstride] = acc[k][v];
+  }
+  __syncthreads();
+  // physical gradient g_c = (sum_d Ja^d_c G_d) / J and the fluxes
+#pragma unroll
+  for (int k = 0; k < PASSES; ++k) {
+    if (!has_node(k)) continue;
+    const int i = tid + k * BLOCK, sl = i / NN, node = i - sl * NN, pn = lds_pos<N>(node);
+    if (sl >= nvalid) continue;
+    const int64_t e = e0 + sl;
+    int id[3];
+    element_indices<DIM>(p, (int)e, id);
+    double ja[DIM][DIM], g[DIM][NV], fv[DIM][NV];
+    node_metric<DIM, N, NODAL, BOX>(p, e, id, node, ja);
+    const double ij = inv_jac<NODAL, NN>(p, e, node);
+#pragma unroll
+    for (int c = 0; c < DIM; ++c) {
+      g[c][0] = 0.0;  // not used by the flux
+#pragma unroll
+      for (int v = 1; v < NV; ++v) {
+        double t = 0.0;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) t += ja[d][c] * s_g[sl * SG + (d * ND + v - 1) * PN + pn];
+        g[c][v] = t * ij;
       }
     }
-    // lower face: this element is primary, (-F_v).(sign(J) Ja^dir) at its node
-    {
-      const double sg = inv_jac<NODAL, NN>(p, e, dofs[0]) >= 0.0 ? 1.0 : -1.0;
-      if (!bnd_lo) {
-        for (int v = 0; v < NV; ++v) acc[0][v] -= sg * f[v * NN + dofs[0]] * p.lhat0;
-      } else {
-        for (int v = vlo[0]; v < vhi[0]; ++v) acc[0][v] -= sg * f[v * NN + dofs[0]] * p.lhat0;
-      }
-    }
-    if (bnd_hi) {
-      const double sg = inv_jac<NODAL, NN>(p, e, dofs[n - 1]) >= 0.0 ? 1.0 : -1.0;
-      for (int v = vlo[1]; v < vhi[1]; ++v) acc[n - 1][v] += sg * f[v * NN + dofs[n - 1]] * p.lhatN;
-    } else {
-      // upper face: the upper neighbour is primary
-      const int64_t nb = p.nbr[e * 2 * DIM + 2 * dir + 1];
-      double s[NV], q[NV], g[DIM][NV], fv[DIM][NV];
-      for (int v = 0; v < NV; ++v) s[v] = p.u[(nb * NV + v) * NN + dofs[0]];
-      grad_vars<DIM>(p.gamma, s, q);
 #pragma unroll
-      for (int c = 0; c < DIM; ++c)
+    for (int c = 0; c < DIM; ++c) viscous_flux_dir<DIM>(p.mu, p.kappa, q[k], g, c, fv[c]);
 #pragma unroll
-        for (int v = 0; v < NV; ++v) g[c][v] = p.grad[((nb * DIM + c) * NV + v) * NN + dofs[0]];
+    for (int d = 0; d < DIM; ++d) {
+      double* out = p.visc_out + (e * DIM + d) * (NV * NN) + row_pos<DIM, N>(d, node);
 #pragma unroll
-      for (int c = 0; c < DIM; ++c) viscous_flux_dir<DIM>(p.mu, p.kappa, q, g, c, fv[c]);
-      double ja[DIM];
-#pragma unroll
-      for (int c = 0; c < DIM; ++c) ja[c] = metric<NODAL, DIM, NN>(p, nb, dir, c, dofs[0]);
-      const double sg = inv_jac<NODAL, NN>(p, nb, dofs[0]) >= 0.0 ? 1.0 : -1.0;
-#pragma unroll
-      for (int v = 0; v < NV; ++v) {
+      for (int v = 1; v < NV; ++v) {
         double r = 0.0;
 #pragma unroll
-        for (int c = 0; c < DIM; ++c) r += ja[c] * -fv[c][v];
-        acc[n - 1][v] += sg * r * p.lhatN;
+        for (int c = 0; c < DIM; ++c) r += ja[d][c] * -fv[c][v];
+        out[v * NN] = r;
       }
     }
-  }
-#pragma unroll
-  for (int d = 0; d < DIM; ++d) {
-    if (valid && dir == d) {
-#pragma unroll
-      for (int k = 0; k < n; ++k)
-#pragma unroll
-        for (int v = 0; v < NV; ++v) {
-          const int idx = (slot * NV + v) * NN + dofs[k];
-          s_du[idx] = d == 0 ? acc[k][v] : s_du[idx] + acc[k][v];
-        }
-    }
-    __syncthreads();
-  }
-  for (int i = tid; i < EPW * NV * NN; i += BLOCK) {
-    if (i / (NV * NN) >= nvalid) continue;
-    p.visc_out[e0 * NV * NN + i] = s_du[i];
   }
 }
 
@@ -470,10 +530,15 @@ hipError_t launch_parabolic_t(bool sc, const KParams& p, hipStream_t s) {
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((gradient_kernel<DIM, N, EPW, NODAL, BCS>), dim3((unsigned)nb), dim3(BLOCK), 0, s, p);
-  hipError_t err = hipGetLastError();
-  if (err != hipSuccess) return err;
-  hipLaunchKernelGGL((viscous_kernel<DIM, N, EPW, NODAL, BCS>), dim3((unsigned)nb), dim3(BLOCK), 0, s, p);
+  if constexpr (NODAL && !BCS) {
+    if (p.ja_box) {
+      hipLaunchKernelGGL((viscous_flux_kernel<DIM, N, EPW, NODAL, BCS, true>), dim3((unsigned)nb),
+                         dim3(BLOCK), 0, s, p);
+      return hipGetLastError();
+    }
+  }
+  hipLaunchKernelGGL((viscous_flux_kernel<DIM, N, EPW, NODAL, BCS, false>), dim3((unsigned)nb),
+                     dim3(BLOCK), 0, s, p);
   return hipGetLastError();
 }
 

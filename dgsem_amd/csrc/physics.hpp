@@ -426,7 +426,7 @@ DG_HD void grad_vars(double gamma, const double* u, double* q) {
 #if defined(__clang__)
 #pragma clang fp contract(off)
 #endif
-  const double inv_rho = 1.0 / u[0];
+  const double inv_rho = div_by(1.0, u[0], recip(u[0]));
   double m2 = 0.0;
   for (int k = 0; k < DIM; ++k) m2 += u[k + 1] * u[k + 1];
   const double p = (gamma - 1.0) * (u[DIM + 1] - 0.5 * m2 * inv_rho);
@@ -443,9 +443,10 @@ DG_HD void viscous_flux_dir(double mu, double kappa, const double* q,
 #if defined(__clang__)
 #pragma clang fp contract(off)
 #endif
+  auto third = [](double x) { return div_by(x, 3.0, 1.0 / 3.0); };
   if constexpr (DIM == 2) {
-    const double tau11 = (4.0 * g[0][1] - 2.0 * g[1][2]) / 3.0;
-    const double tau22 = (4.0 * g[1][2] - 2.0 * g[0][1]) / 3.0;
+    const double tau11 = third(4.0 * g[0][1] - 2.0 * g[1][2]);
+    const double tau22 = third(4.0 * g[1][2] - 2.0 * g[0][1]);
     const double tau12 = g[1][1] + g[0][2];
     const double t1 = dim == 0 ? tau11 : tau12, t2 = dim == 0 ? tau12 : tau22;
     f[0] = 0.0;
@@ -453,9 +454,9 @@ DG_HD void viscous_flux_dir(double mu, double kappa, const double* q,
     f[2] = mu * t2;
     f[3] = mu * (q[1] * t1 + q[2] * t2 + kappa * g[dim][3]);
   } else {
-    const double tau11 = (4.0 * g[0][1] - 2.0 * (g[1][2] + g[2][3])) / 3.0;
-    const double tau22 = (4.0 * g[1][2] - 2.0 * (g[0][1] + g[2][3])) / 3.0;
-    const double tau33 = (4.0 * g[2][3] - 2.0 * (g[0][1] + g[1][2])) / 3.0;
+    const double tau11 = third(4.0 * g[0][1] - 2.0 * (g[1][2] + g[2][3]));
+    const double tau22 = third(4.0 * g[1][2] - 2.0 * (g[0][1] + g[2][3]));
+    const double tau33 = third(4.0 * g[2][3] - 2.0 * (g[0][1] + g[1][2]));
     const double tau12 = g[1][1] + g[0][2];
     const double tau13 = g[2][1] + g[0][3];
     const double tau23 = g[2][2] + g[1][3];
