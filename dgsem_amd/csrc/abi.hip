@@ -66,10 +66,8 @@ void release(dgsem_handle* h) {
   hipFree(h->d_Vinv);
   hipFree(h->d_ja_box);
   hipFree(h->d_alpha);
-  hipFree(h->d_grad);
   hipFree(h->d_visc);
   hipFree(h->d_ad_dgrad);
-  hipFree(h->d_ad_dvisc);
   hipFree(h->d_ad_qbar);
   hipFree(h->d_wq);
   hipFree(h->d_ke_partial);
@@ -78,9 +76,9 @@ void release(dgsem_handle* h) {
   hipFree(h->d_ad_out);
   hipFree(h->d_fl_r);
   hipFree(h->d_fl_w);
-  h->d_ad_dgrad = h->d_ad_dvisc = h->d_ad_qbar = h->d_wq = h->d_ke_partial = nullptr;
+  h->d_ad_dgrad = h->d_ad_qbar = h->d_wq = h->d_ke_partial = nullptr;
   h->d_an_partial = h->d_ad_alpha = h->d_ad_out = h->d_fl_r = h->d_fl_w = nullptr;
-  h->d_Ja = h->d_invJ = h->d_sn = h->d_Vinv = h->d_alpha = h->d_grad = h->d_visc = nullptr;
+  h->d_Ja = h->d_invJ = h->d_sn = h->d_Vinv = h->d_alpha = h->d_visc = nullptr;
   h->d_nbr = nullptr;
   h->d_ja_box = nullptr;
 }
@@ -188,8 +186,6 @@ void fill_params(dgsem_handle* h) {
   // Navier-Stokes: kappa = gamma / ((gamma - 1) Pr), compressible_navier_stokes3D.hpp:19-22
   p.mu = c.mu;
   p.kappa = c.gamma / ((c.gamma - 1.0) * c.prandtl);
-  p.grad = h->d_grad;
-  p.grad_out = h->d_grad;
   p.visc_out = h->d_visc;
   for (int k = 0; k < 3; ++k) p.cells[k] = c.cells[k];
   p.div_y = dgsem::FastDiv::by((uint32_t)c.cells[1]);
@@ -402,17 +398,12 @@ int dgsem_create(const dgsem_config* cfg, void* stream, dgsem_handle** out) {
   std::vector<double> sn;
   if (h->cfg.geometry == DGSEM_GEOMETRY_NODAL && h->cfg.volume_integral == DGSEM_VOLUME_SHOCK_CAPTURING)
     sn = h->geo.subcell_normals;
-  const bool node_kernel = dgsem::node_kernel_for(
-      h->cfg.polydeg, h->cfg.volume_integral == DGSEM_VOLUME_SHOCK_CAPTURING, has_boundaries(h->cfg));
   if ((rc = upload(h, &h->d_Ja, Ja)) || (rc = upload(h, &h->d_invJ, invJ)) ||
       (rc = upload(h, &h->d_sn, sn)) || (rc = upload(h, &h->d_nbr, neighbour_table(h->geo, periodic))) ||
       (rc = upload(h, &h->d_Vinv, h->basis.Vinv)) ||
       (rc = upload(h, &h->d_alpha, std::vector<double>(4 * h->E, 0.0))) ||
-      // Navier-Stokes: the viscous fluxes, and the gradient of the tangent and
-      // adjoint (which allocate it themselves where the node kernel runs)
       (h->cfg.equation == DGSEM_NAVIER_STOKES &&
-       ((!node_kernel && (rc = alloc_zero(h, &h->d_grad, (size_t)h->E * h->cfg.dim * h->nvars * h->nn))) ||
-        (rc = alloc_zero(h, &h->d_visc, (size_t)h->E * h->cfg.dim * h->nvars * h->nn))))) {
+       (rc = alloc_zero(h, &h->d_visc, (size_t)h->E * h->cfg.dim * h->nvars * h->nn)))) {
     release(h);
     *out = h;
     return rc;

@@ -58,28 +58,6 @@ hipError_t launch_vjp(int dim, int N, bool nodal, bool ns, const AdParams& a, hi
   }
 }
 
-hipError_t launch_gradient(int dim, int N, bool nodal, const KParams& p, hipStream_t s) {
-  if (dim == 2) {
-    switch (N) {
-      case 1: return launch_gradient_dn<2, 1>(nodal, p, s);
-      case 2: return launch_gradient_dn<2, 2>(nodal, p, s);
-      case 3: return launch_gradient_dn<2, 3>(nodal, p, s);
-      case 4: return launch_gradient_dn<2, 4>(nodal, p, s);
-      case 5: return launch_gradient_dn<2, 5>(nodal, p, s);
-      case 7: return launch_gradient_dn<2, 7>(nodal, p, s);
-      default: return hipErrorInvalidValue;
-    }
-  }
-  switch (N) {
-    case 2: return launch_gradient_dn<3, 2>(nodal, p, s);
-    case 3: return launch_gradient_dn<3, 3>(nodal, p, s);
-    case 4: return launch_gradient_dn<3, 4>(nodal, p, s);
-    case 5: return launch_gradient_dn<3, 5>(nodal, p, s);
-    case 7: return launch_gradient_dn<3, 7>(nodal, p, s);
-    default: return hipErrorInvalidValue;
-  }
-}
-
 namespace {
 
 constexpr int kKeBlock = 256;
@@ -211,13 +189,7 @@ int ad_prepare(dgsem_handle* h) {
   }
   if (c.equation == DGSEM_NAVIER_STOKES) {
     int rc;
-    // the forward gradient, which the node-parallel forward path never stores
-    if (!h->d_grad) {
-      if ((rc = alloc_once(h, &h->d_grad, cell * c.dim))) return rc;
-      h->base.grad = h->base.grad_out = h->d_grad;
-    }
-    if ((rc = alloc_once(h, &h->d_ad_dgrad, cell * c.dim)) ||
-        (rc = alloc_once(h, &h->d_ad_dvisc, cell)) || (rc = alloc_once(h, &h->d_ad_qbar, cell)))
+    if ((rc = alloc_once(h, &h->d_ad_dgrad, cell * c.dim)) || (rc = alloc_once(h, &h->d_ad_qbar, cell)))
       return rc;
   }
   return DGSEM_OK;
@@ -227,10 +199,7 @@ dgsem::AdParams ad_params(dgsem_handle* h, const double* u) {
   dgsem::AdParams a{};
   a.k = h->base;
   a.k.u = u;
-  a.k.grad = h->d_grad;
-  a.k.grad_out = h->d_grad;
-  a.dgrad = h->d_ad_dgrad;
-  a.dvisc = h->cfg.equation == DGSEM_NAVIER_STOKES ? h->d_ad_dvisc : nullptr;
+  a.dgrad = h->cfg.equation == DGSEM_NAVIER_STOKES ? h->d_ad_dgrad : nullptr;
   a.qbar = h->d_ad_qbar;
   return a;
 }
@@ -263,12 +232,8 @@ int apply(dgsem_handle* h, bool adjoint, const double* u, const double* v, const
   a.b = b;
   a.c = c;
   a.out = out;
-  hipError_t e;
-  if (ns) {
-    e = dgsem::launch_gradient(h->cfg.dim, h->cfg.polydeg, nodal, a.k, h->stream);
-    if (e != hipSuccess) return ahip(h, e, "gradient kernel launch");
-  }
-  e = adjoint ? dgsem::launch_vjp(h->cfg.dim, h->cfg.polydeg, nodal, ns, a, h->stream)
+  const hipError_t e =
+      adjoint ? dgsem::launch_vjp(h->cfg.dim, h->cfg.polydeg, nodal, ns, a, h->stream)
               : dgsem::launch_jvp(h->cfg.dim, h->cfg.polydeg, nodal, ns, a, h->stream);
   return e == hipSuccess ? DGSEM_OK : ahip(h, e, adjoint ? "adjoint kernel launch" : "tangent kernel launch");
 }

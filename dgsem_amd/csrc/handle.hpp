@@ -29,16 +29,12 @@ struct dgsem_handle {
   double* d_alpha = nullptr;  // blending factor per element, [4][E]: slot 0 the last
                               // dgsem_rhs, slots 1-3 the last SSPRK3 stage of each kind
   int alpha_last = 0;         // slot of the last launch that wrote one
-  double* d_grad = nullptr;  // Navier-Stokes gradient [E][dim][var][dof], for the
-                             // tangent and adjoint
   double* d_visc = nullptr;  // Navier-Stokes viscous fluxes [E][dim][var][NN]
   dgsem::KParams base{};
   // tangent / adjoint scratch, allocated on first use: d_ad_dgrad
-  // [E][dim][NV][NN], d_ad_dvisc and d_ad_qbar [E][NV][NN] (Navier-Stokes),
-  // d_wq the tensor-product quadrature weight of each node, d_ke_partial the
+  // [E][dim][NV][NN] and d_ad_qbar [E][NV][NN] (Navier-Stokes), d_wq the tensor-product quadrature weight of each node, d_ke_partial the
   // per-block sums of the kinetic-energy reduction
   double* d_ad_dgrad = nullptr;
-  double* d_ad_dvisc = nullptr;
   double* d_ad_qbar = nullptr;
   double* d_wq = nullptr;
   double* d_ke_partial = nullptr;

@@ -77,8 +77,6 @@ struct KParams {
   const double* sn;      // nodal subcell normals [E][dim][FN][N][dim]
   const int* nbr;        // [E][2*dim] (lower, upper) neighbour per direction
   const double* Vinv;    // [n][n] inverse Legendre Vandermonde
-  const double* grad;    // Navier-Stokes: gradient [E][dim][var][dof]
-  double* grad_out;      // written by the gradient kernel
   const double* visc;    // Navier-Stokes: viscous fluxes (parabolic_impl.hpp)
   double* visc_out;      // written by the viscous kernel
   int64_t E;
@@ -139,8 +137,8 @@ hipError_t launch_pack_left(const double* src, double* dst, const int cells[3], 
 // kernels write
 //     out = a1 x1 + a2 x2 + b v + c Op(v)
 // (x1, x2 may be null), which covers the tangent and adjoint of every SSPRK3
-// stage.  Navier-Stokes needs k.grad = the forward gradient of k.u and the
-// scratch arrays dgrad [E][dim][NV][NN], dvisc and qbar [E][NV][NN].
+// stage.  Navier-Stokes needs the scratch arrays dgrad [E][dim][NV][NN] (null
+// for Euler) and qbar [E][NV][NN].
 struct AdParams {
   KParams k;
   const double* v;  // tangent direction or cotangent
@@ -149,7 +147,6 @@ struct AdParams {
   double a1, a2, b, c;
   double* out;
   double* dgrad;
-  double* dvisc;
   double* qbar;
 };
 
@@ -157,17 +154,11 @@ template <int DIM, int N>
 hipError_t launch_jvp_dn(bool nodal, const AdParams& a, hipStream_t stream);
 template <int DIM, int N>
 hipError_t launch_vjp_dn(bool nodal, const AdParams& a, hipStream_t stream);
-// Launch the tangent or adjoint kernels for (dim, N); the Navier-Stokes
-// forward gradient must already be in a.k.grad.
+// Launch the tangent or adjoint kernels for (dim, N).
 hipError_t launch_jvp(int dim, int N, bool nodal, bool navier_stokes, const AdParams& a,
                       hipStream_t stream);
 hipError_t launch_vjp(int dim, int N, bool nodal, bool navier_stokes, const AdParams& a,
                       hipStream_t stream);
-// Forward BR1 gradient alone (a.k.grad_out from a.k.u).
-template <int DIM, int N>
-hipError_t launch_gradient_dn(bool nodal, const KParams& p, hipStream_t stream);
-hipError_t launch_gradient(int dim, int N, bool nodal, const KParams& p, hipStream_t stream);
-
 // Kinetic energy sum_e sum_i w_i / |1/J_i| |m_i|^2 / (2 rho_i) into *result
 // (device), and its gradient: grad += scale * dKE/du.  partial: scratch of
 // ke_partials(E) doubles.

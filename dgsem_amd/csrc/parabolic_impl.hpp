@@ -18,8 +18,8 @@
 //     so that a line thread reads contiguous runs.
 //   * gradient_node_kernel: for the elements of the node-parallel RHS kernel
 //     (node_kernel_for), rounded as the reference; layout [E][d][var][dof].
-// gradient_kernel writes the gradient [E][dim][var][dof] for the tangent and
-// adjoint kernels.
+// The tangent and adjoint kernels (adjoint_impl.hpp) form the gradient they
+// linearise at themselves, with line_gradient.
 // BCS (2D): some face is not periodic; the neighbour table holds -1 there and
 // the face values come from the boundary condition (wall_gradient_value and
 // rhs_kernel's wall branch).
@@ -84,112 +84,6 @@ __device__ __forceinline__ void wall_gradient_value(int kind, const double* q, c
   }
 }
 
-template <int DIM, int N, int EPW, bool NODAL, bool BCS>
-__global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) gradient_kernel(const KParams p) {
-  using S = Shape<DIM, N>;
-  constexpr int n = S::n, NV = S::NV, NN = S::NN, FN = S::FN, L = S::LINES;
-  constexpr int BLOCK = EPW * L;
-  __shared__ double s_q[EPW * NV * NN];
-  __shared__ double s_g[EPW * DIM * NV * NN];  // per direction: D_hat q + lift
-  const int tid = threadIdx.x;
-  const int blk = xcd_block(blockIdx.x, gridDim.x);
-  const int64_t e0 = (int64_t)blk * EPW;
-  const int nvalid = (int)((p.E - e0) < EPW ? (p.E - e0) : EPW);
-
-  for (int i = tid; i < EPW * NN; i += BLOCK) {
-    const int sl = i / NN, node = i % NN;
-    if (sl >= nvalid) continue;
-    double s[NV], q[NV];
-    for (int v = 0; v < NV; ++v) s[v] = p.u[((e0 + sl) * NV + v) * NN + node];
-    grad_vars<DIM>(p.gamma, s, q);
-    for (int v = 0; v < NV; ++v) s_q[(sl * NV + v) * NN + node] = q[v];
-  }
-  __syncthreads();
-
-  const int slot = tid / L, rem = tid % L, dir = rem / FN, line = rem % FN;
-  if (slot < nvalid) {
-    const int64_t e = e0 + slot;
-    int dofs[n];
-#pragma unroll
-    for (int k = 0; k < n; ++k) dofs[k] = line_dof<DIM, N>(dir, line, k);
-    const double* q = s_q + slot * NV * NN;
-    double acc[n][NV];
-#pragma unroll
-    for (int k = 0; k < n; ++k)
-#pragma unroll
-      for (int v = 0; v < NV; ++v) {
-        double r = 0.0;
-#pragma unroll
-        for (int i = 0; i < n; ++i) r += p.Dhat[k][i] * q[v * NN + dofs[i]];
-        acc[k][v] = r;
-      }
-    // BR1 face values q_hat = (q_lower + q_upper) / 2 on both line ends
-#pragma unroll 1
-    for (int side = 0; side < 2; ++side) {
-      const int64_t nb = p.nbr[e * 2 * DIM + 2 * dir + side];
-      if constexpr (BCS) {
-        if (nb < 0) {
-          const int dof_own = side == 0 ? dofs[0] : dofs[n - 1];
-          const double sg = inv_jac<NODAL, NN>(p, e, dof_own) >= 0.0 ? 1.0 : -1.0;
-          double qo[NV], nrm[DIM], qw[NV];
-          const int face = 2 * dir + side;
-          if (p.bc[face] == kBcDirichlet) {
-            const int64_t along = dir == 0 ? e % p.cells[1] : e / p.cells[1];
-            const int64_t bnode = along * n + line;
-            const double* vals = p.bc_values[face];
-            double so[NV];
-            for (int v = 0; v < NV; ++v) so[v] = vals ? vals[bnode * NV + v] : p.bc_state[face][v];
-            grad_vars<DIM>(p.gamma, so, qw);
-          } else {
-            for (int v = 0; v < NV; ++v) qo[v] = q[v * NN + dof_own];
-            for (int c = 0; c < DIM; ++c) nrm[c] = sg * metric<NODAL, DIM, NN>(p, e, dir, c, dof_own);
-            wall_gradient_value<DIM>(p.bc[face], qo, nrm, qw);
-          }
-          if (side == 0) {
-            for (int v = 0; v < NV; ++v) acc[0][v] -= sg * p.lhat0 * qw[v];
-          } else {
-            for (int v = 0; v < NV; ++v) acc[n - 1][v] += sg * p.lhatN * qw[v];
-          }
-          continue;
-        }
-      }
-      const int dof_nb = side == 0 ? dofs[n - 1] : dofs[0];
-      double s[NV], qn[NV];
-      for (int v = 0; v < NV; ++v) s[v] = p.u[(nb * NV + v) * NN + dof_nb];
-      grad_vars<DIM>(p.gamma, s, qn);
-      // the face term uses the element's own normal sign(J) Ja^dir at its node
-      const int dof_own = side == 0 ? dofs[0] : dofs[n - 1];
-      const double sg = inv_jac<NODAL, NN>(p, e, dof_own) >= 0.0 ? 1.0 : -1.0;
-      if (side == 0) {
-        for (int v = 0; v < NV; ++v) acc[0][v] -= sg * p.lhat0 * (0.5 * (qn[v] + q[v * NN + dofs[0]]));
-      } else {
-        for (int v = 0; v < NV; ++v) acc[n - 1][v] += sg * p.lhatN * (0.5 * (q[v * NN + dofs[n - 1]] + qn[v]));
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < n; ++k)
-#pragma unroll
-      for (int v = 0; v < NV; ++v) s_g[((slot * DIM + dir) * NV + v) * NN + dofs[k]] = acc[k][v];
-  }
-  __syncthreads();
-  // physical gradient: g_c = (sum_d Ja^d_c G_d) / J
-  for (int i = tid; i < EPW * NN; i += BLOCK) {
-    const int sl = i / NN, node = i % NN;
-    if (sl >= nvalid) continue;
-    const int64_t e = e0 + sl;
-    const double ij = inv_jac<NODAL, NN>(p, e, node);
-    for (int c = 0; c < DIM; ++c) {
-      double ja[DIM];
-      for (int d = 0; d < DIM; ++d) ja[d] = metric<NODAL, DIM, NN>(p, e, d, c, node);
-      for (int v = 0; v < NV; ++v) {
-        double g = 0.0;
-        for (int d = 0; d < DIM; ++d) g += ja[d] * s_g[((sl * DIM + d) * NV + v) * NN + node];
-        p.grad_out[((e * DIM + c) * NV + v) * NN + node] = g * ij;
-      }
-    }
-  }
-}
-
 // Position of node `dof` in the direction-d rows line * n + k (LineNodes).
 template <int DIM, int N>
 __device__ __forceinline__ int row_pos(int d, int dof) {
@@ -212,6 +106,60 @@ __device__ __forceinline__ void node_metric(const KParams& p, int64_t e, const i
     for (int c = 0; c < DIM; ++c)
       ja[d][c] = BOX ? 2.0 * box_row<DIM, N>(p, eid, c, d, 0)[row_pos<DIM, N>(d, dof)]
                      : metric<NODAL, DIM, NN>(p, e, d, c, dof);
+}
+
+// The weak derivative of the variables v, T along one line, with the BR1 face
+// values lifted: acc = D_hat x -+ l_hat sign(J) q_hat, q_hat = (q_L + q_R) / 2 on
+// both line ends.  x[k][v - 1]: the line's variables; q_lo, q_hi: the
+// neighbours' (NV values, from grad_vars; overwritten); blo, bhi: the end is a
+// boundary face, whose value comes from the boundary condition; sg_*: sign(J) at
+// the line's end nodes (the face terms use the element's own normal).
+template <int DIM, int N, bool NODAL, bool BCS>
+__device__ __forceinline__ void line_gradient(const KParams& p, int64_t el, const int* eid, int dl,
+                                              int line, int first, int last,
+                                              const double (&x)[N + 1][DIM + 1], double* q_lo,
+                                              double* q_hi, bool blo, bool bhi, double sg_lo,
+                                              double sg_hi, double (&acc)[N + 1][DIM + 1]) {
+  constexpr int n = N + 1, NV = DIM + 2, ND = NV - 1, NN = Shape<DIM, N>::NN;
+#pragma unroll
+  for (int k = 0; k < n; ++k)
+#pragma unroll
+    for (int v = 0; v < ND; ++v) {
+      double r = 0.0;
+#pragma unroll
+      for (int i = 0; i < n; ++i) r += p.Dhat[k][i] * x[i][v];
+      acc[k][v] = r;
+    }
+#pragma unroll
+  for (int v = 1; v < NV; ++v) {
+    q_lo[v] = 0.5 * (q_lo[v] + x[0][v - 1]);
+    q_hi[v] = 0.5 * (x[n - 1][v - 1] + q_hi[v]);
+  }
+  if constexpr (BCS) {
+    auto wall = [&](int side, int dof, double sg, const double* xn, double* out) {
+      const int face = 2 * dl + side;
+      if (p.bc[face] == kBcDirichlet) {
+        const int64_t bnode = (int64_t)(dl == 0 ? eid[1] : eid[0]) * n + line;
+        const double* vals = p.bc_values[face];
+        double so[NV];
+        for (int v = 0; v < NV; ++v) so[v] = vals ? vals[bnode * NV + v] : p.bc_state[face][v];
+        grad_vars<DIM>(p.gamma, so, out);
+      } else {
+        double own[NV], nrm[DIM];
+        own[0] = 0.0;  // rho: not differentiated
+        for (int v = 1; v < NV; ++v) own[v] = xn[v - 1];
+        for (int c = 0; c < DIM; ++c) nrm[c] = sg * metric<NODAL, DIM, NN>(p, el, dl, c, dof);
+        wall_gradient_value<DIM>(p.bc[face], own, nrm, out);
+      }
+    };
+    if (blo) wall(0, first, sg_lo, x[0], q_lo);
+    if (bhi) wall(1, last, sg_hi, x[n - 1], q_hi);
+  }
+#pragma unroll
+  for (int v = 1; v < NV; ++v) {
+    acc[0][v - 1] -= sg_lo * p.lhat0 * q_lo[v];
+    acc[n - 1][v - 1] += sg_hi * p.lhatN * q_hi[v];
+  }
 }
 
 // The nodes' viscous fluxes into p.visc_out (see the top of the file).  Memory
@@ -269,7 +217,6 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) viscous_flux_ker
       t_hi[v] = uhi[v * NN];
     }
   }
-  // the face terms use the element's own normal sign(J) Ja^dir at its nodes
   const double sg_lo = BOX || inv_jac<NODAL, NN>(p, el, first) >= 0.0 ? 1.0 : -1.0;
   const double sg_hi = BOX || inv_jac<NODAL, NN>(p, el, last) >= 0.0 ? 1.0 : -1.0;
 #pragma unroll
@@ -292,49 +239,11 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) viscous_flux_ker
     for (int k = 0; k < n; ++k)
 #pragma unroll
       for (int v = 0; v < ND; ++v) x[k][v] = s_g[slot * SG + v * PN + ln.pbase + k * ln.pstride];
-#pragma unroll
-    for (int k = 0; k < n; ++k)
-#pragma unroll
-      for (int v = 0; v < ND; ++v) {
-        double r = 0.0;
-#pragma unroll
-        for (int i = 0; i < n; ++i) r += p.Dhat[k][i] * x[i][v];
-        acc[k][v] = r;
-      }
-    // BR1 face values q_hat = (q_lower + q_upper) / 2 on both line ends
     double q_lo[NV], q_hi[NV];
     grad_vars<DIM>(p.gamma, t_lo, q_lo);
     grad_vars<DIM>(p.gamma, t_hi, q_hi);
-#pragma unroll
-    for (int v = 1; v < NV; ++v) {
-      q_lo[v] = 0.5 * (q_lo[v] + x[0][v - 1]);
-      q_hi[v] = 0.5 * (x[n - 1][v - 1] + q_hi[v]);
-    }
-    if constexpr (BCS) {
-      auto wall = [&](int side, int dof, double sg, const double* xn, double* out) {
-        const int face = 2 * dl + side;
-        if (p.bc[face] == kBcDirichlet) {
-          const int64_t bnode = (int64_t)(dl == 0 ? eid[1] : eid[0]) * n + line;
-          const double* vals = p.bc_values[face];
-          double so[NV];
-          for (int v = 0; v < NV; ++v) so[v] = vals ? vals[bnode * NV + v] : p.bc_state[face][v];
-          grad_vars<DIM>(p.gamma, so, out);
-        } else {
-          double own[NV], nrm[DIM];
-          own[0] = 0.0;  // rho: not differentiated
-          for (int v = 1; v < NV; ++v) own[v] = xn[v - 1];
-          for (int c = 0; c < DIM; ++c) nrm[c] = sg * metric<NODAL, DIM, NN>(p, el, dl, c, dof);
-          wall_gradient_value<DIM>(p.bc[face], own, nrm, out);
-        }
-      };
-      if (blo) wall(0, first, sg_lo, x[0], q_lo);
-      if (bhi) wall(1, last, sg_hi, x[n - 1], q_hi);
-    }
-#pragma unroll
-    for (int v = 1; v < NV; ++v) {
-      acc[0][v - 1] -= sg_lo * p.lhat0 * q_lo[v];
-      acc[n - 1][v - 1] += sg_hi * p.lhatN * q_hi[v];
-    }
+    line_gradient<DIM, N, NODAL, BCS>(p, el, eid, dl, line, first, last, x, q_lo, q_hi, blo, bhi,
+                                      sg_lo, sg_hi, acc);
   }
   __syncthreads();  // every line has read its q
   if (dir < DIM) {

@@ -30,7 +30,7 @@ struct PrimTangent {
 template <int DIM>
 DG_HD void prims_jvp(double gamma, const double* u, const NodePrims<DIM>& q, const double* du,
                      PrimTangent<DIM>& dq) {
-  const double ir = 1.0 / q.rho;
+  const double ir = recip(q.rho);
   dq.rho = du[0];
   double dkin = 0.0;
   for (int k = 0; k < DIM; ++k) {
@@ -39,7 +39,7 @@ DG_HD void prims_jvp(double gamma, const double* u, const NodePrims<DIM>& q, con
   }
   dq.kin = dkin;
   const double dp = (gamma - 1.0) * (du[DIM + 1] - q.kin * du[0] - q.rho * dkin);
-  dq.beta = q.beta * (du[0] * ir - dp / q.p);
+  dq.beta = q.beta * (du[0] * ir - dp * recip(q.p));
   (void)u;
 }
 
@@ -47,9 +47,9 @@ DG_HD void prims_jvp(double gamma, const double* u, const NodePrims<DIM>& q, con
 template <int DIM>
 DG_HD void prims_vjp(double gamma, const NodePrims<DIM>& q, const PrimTangent<DIM>& qbar,
                      double pbar, double* ubar) {
-  const double ir = 1.0 / q.rho;
+  const double ir = recip(q.rho);
   double rb = qbar.rho + qbar.beta * q.beta * ir;
-  double pb = pbar - qbar.beta * q.beta / q.p;
+  double pb = pbar - qbar.beta * q.beta * recip(q.p);
   double vb[DIM];
   for (int k = 0; k < DIM; ++k) vb[k] = qbar.v[k] + qbar.kin * q.v[k];
   // p = (gamma - 1) (E - rho kin(v)), with v held as an independent variable
@@ -64,35 +64,36 @@ DG_HD void prims_vjp(double gamma, const NodePrims<DIM>& q, const PrimTangent<DI
   ubar[0] += rb;
 }
 
-// Logarithmic mean and its partial derivatives on both branches, the one
-// the forward evaluation took selected by `series`.  Both are computed and
-// one is selected without a branch: divergent branches in each of the
-// unrolled pair evaluations of a line would keep the line's state live across
-// all of them and multiply the register count.  On the series branch the log
-// form may be inf / nan (x == y); it is discarded by the select.
-DG_HD void ln_mean_partials(double x, double y, bool series, double& L, double& Lx, double& Ly) {
-  const double s = x + y, d = x - y;
-  const double is = 1.0 / s;
-  const double f = d * d * is * is;
-  const double P = 2.0 + f * (2.0 / 3.0 + f * (2.0 / 5.0 + f * (2.0 / 7.0)));
-  const double dP = 2.0 / 3.0 + f * (4.0 / 5.0 + f * (6.0 / 7.0));
-  const double fx = 2.0 * d * is * is - 2.0 * d * d * is * is * is;
-  const double fy = -2.0 * d * is * is - 2.0 * d * d * is * is * is;
-  const double Ls = s / P;
-  const double c = s * dP / (P * P);
-  const double Lxs = 1.0 / P - c * fx, Lys = 1.0 / P - c * fy;
-  const double D = log(y / x);
-  const double Ll = (y - x) / D;
-  const double Lxl = (Ll / x - 1.0) / D, Lyl = (1.0 - Ll / y) / D;
-  L = series ? Ls : Ll;
-  Lx = series ? Lxs : Lxl;
-  Ly = series ? Lys : Lyl;
+// Q = artanh(xi) / xi of a pair (physics.hpp) and dQ/df2, f2 = xi^2: the series
+// and its derivative term by term, or the identity dQ/df2 = (1 / (1 - f2) - Q) /
+// (2 f2) with 1 - f2 = 4 x y / (x + y)^2.
+DG_HD void artanh_ratio_jet(double x, double y, double f2, double& Q, double& dQ) {
+  Q = artanh_ratio(x, y, f2);
+  if (f2 < kSeriesMax) {
+    double d = 10.0 / 21.0;
+    d = 9.0 / 19.0 + f2 * d;
+    d = 8.0 / 17.0 + f2 * d;
+    d = 7.0 / 15.0 + f2 * d;
+    d = 6.0 / 13.0 + f2 * d;
+    d = 5.0 / 11.0 + f2 * d;
+    d = 4.0 / 9.0 + f2 * d;
+    d = 3.0 / 7.0 + f2 * d;
+    d = 2.0 / 5.0 + f2 * d;
+    dQ = 1.0 / 3.0 + f2 * d;
+  } else {
+    const double s = x + y;
+    dQ = (s * s * recip(4.0 * x * y) - Q) * recip(2.0 * f2);
+  }
 }
 
 // Means of the Chandrashekar flux and their partial derivatives with
 // respect to (rho_a, rho_b) and (beta_a, beta_b): rho_mean, its inverse
 // beta mean B = 1 / ln_mean(beta_a, beta_b) and p_mean = (rho_a + rho_b) /
-// (2 (beta_a + beta_b)).  The branch test is the forward's.
+// (2 (beta_a + beta_b)), as flux_chandrashekar forms them, with its branches.
+// rho_mean = s / 2 P and B = 2 Q / s; xi_x = 2 y / s^2, xi_y = -2 x / s^2.  With
+// both branches and IEEE quotients evaluated for every pair (selected without a
+// branch) the derivative kernels spent four times the FP64 instructions; their
+// callers pin the sums after each pair, so the branch costs no registers.
 struct ChandrashekarMeans {
   double rho, rho_a, rho_b;  // rho_mean and partials
   double B, B_a, B_b;        // inverse beta mean and partials
@@ -102,98 +103,95 @@ struct ChandrashekarMeans {
 template <int DIM>
 DG_HD ChandrashekarMeans chandrashekar_means(const NodePrims<DIM>& a, const NodePrims<DIM>& b) {
   const double sr = a.rho + b.rho, sb = a.beta + b.beta;
-  const double xr = a.rho - b.rho, xb = a.beta - b.beta;
-  const double nr = xr * xr, dr = sr * sr;
-  const double nb = xb * xb, db = sb * sb;
-  const double r1 = 1.0 / (dr * db);
-  const double f2r = nr * (db * r1), f2b = nb * (dr * r1);
+  const double r = recip(sr * sb);
+  const double isr = r * sb, isb = r * sr;
+  const double xr = (a.rho - b.rho) * isr, xb = (a.beta - b.beta) * isb;
+  const double fr = xr * xr, fb = xb * xb;
+  double P, dP, Q, dQ;  // functions of f2 and their derivatives
+  if (fr < 1.0e-4 && fb < 1.0e-4) {
+    P = 1.0 - fr * (1.0 / 3.0 + fr * (4.0 / 45.0 + fr * (44.0 / 945.0)));
+    dP = -(1.0 / 3.0 + fr * (8.0 / 45.0 + fr * (44.0 / 315.0 + fr * (1712.0 / 14175.0))));
+    Q = 1.0 + fb * (1.0 / 3.0 + fb * (1.0 / 5.0 + fb * (1.0 / 7.0)));
+    dQ = 1.0 / 3.0 + fb * (2.0 / 5.0 + fb * (3.0 / 7.0 + fb * (4.0 / 9.0)));
+  } else {
+    artanh_ratio_jet(a.rho, b.rho, fr, P, dP);
+    P = recip(P);
+    dP = -dP * P * P;
+    artanh_ratio_jet(a.beta, b.beta, fb, Q, dQ);
+  }
   ChandrashekarMeans m;
-  ln_mean_partials(a.rho, b.rho, f2r < 1.0e-4, m.rho, m.rho_a, m.rho_b);
-  double Lb, Lba, Lbb;
-  ln_mean_partials(a.beta, b.beta, f2b < 1.0e-4, Lb, Lba, Lbb);
-  m.B = 1.0 / Lb;
-  m.B_a = -m.B * m.B * Lba;
-  m.B_b = -m.B * m.B * Lbb;
-  m.p = 0.5 * sr / sb;
-  m.p_rho = 0.5 / sb;
-  m.p_beta = -m.p / sb;
+  m.rho = 0.5 * sr * P;
+  const double t = 2.0 * xr * isr * dP;
+  m.rho_a = 0.5 * P + t * b.rho;
+  m.rho_b = 0.5 * P - t * a.rho;
+  m.B = 2.0 * isb * Q;
+  const double c = 2.0 * isb * isb, w = 4.0 * xb * isb * dQ;
+  m.B_a = c * (w * b.beta - Q);
+  m.B_b = -c * (w * a.beta + Q);
+  m.p = 0.5 * sr * isb;
+  m.p_rho = 0.5 * isb;
+  m.p_beta = -m.p * isb;
   return m;
 }
 
 // Tangent of the Chandrashekar flux with respect to both nodes' primitives
-// (the normal n is geometry, not differentiated).
+// (the normal n is geometry, not differentiated), in flux_chandrashekar's form:
+// f = (2 h, h vs + p n, h (B / (gamma - 1) + v_a . v_b) + p vn / 2) with vs =
+// v_a + v_b, vn = vs . n and h = rho_mean vn / 4.
 template <int DIM>
 DG_HD void chandrashekar_jvp(double inv_gm1, const NodePrims<DIM>& a, const NodePrims<DIM>& b,
                              const PrimTangent<DIM>& da, const PrimTangent<DIM>& db,
                              const double* n, double* df) {
   const ChandrashekarMeans m = chandrashekar_means<DIM>(a, b);
-  double vna = 0.0, vnb = 0.0, dvna = 0.0, dvnb = 0.0;
+  double vs[DIM], dvs[DIM], vn = 0.0, dvn = 0.0, dot = 0.0, ddot = 0.0;
   for (int k = 0; k < DIM; ++k) {
-    vna += a.v[k] * n[k];
-    vnb += b.v[k] * n[k];
-    dvna += da.v[k] * n[k];
-    dvnb += db.v[k] * n[k];
+    vs[k] = a.v[k] + b.v[k];
+    dvs[k] = da.v[k] + db.v[k];
+    vn += vs[k] * n[k];
+    dvn += dvs[k] * n[k];
+    dot += a.v[k] * b.v[k];
+    ddot += da.v[k] * b.v[k] + a.v[k] * db.v[k];
   }
   const double drm = m.rho_a * da.rho + m.rho_b * db.rho;
   const double dB = m.B_a * da.beta + m.B_b * db.beta;
-  const double dpm = m.p_rho * (da.rho + db.rho) + m.p_beta * (da.beta + db.beta);
-  const double vsq = a.kin + b.kin, dvsq = da.kin + db.kin;
-  const double f1 = m.rho * 0.5 * (vna + vnb);
-  const double df1 = drm * 0.5 * (vna + vnb) + m.rho * 0.5 * (dvna + dvnb);
-  const double A = 0.5 * (inv_gm1 * m.B - vsq);
-  double dfe = df1 * A + f1 * 0.5 * (inv_gm1 * dB - dvsq);
-  df[0] = df1;
-  for (int k = 0; k < DIM; ++k) {
-    const double vavg = 0.5 * (a.v[k] + b.v[k]);
-    const double dvavg = 0.5 * (da.v[k] + db.v[k]);
-    const double fk = f1 * vavg + m.p * n[k];
-    const double dfk = df1 * vavg + f1 * dvavg + dpm * n[k];
-    df[k + 1] = dfk;
-    dfe += dfk * vavg + fk * dvavg;
-  }
-  df[DIM + 1] = dfe;
+  const double dp = m.p_rho * (da.rho + db.rho) + m.p_beta * (da.beta + db.beta);
+  const double h = 0.25 * m.rho * vn;
+  const double dh = 0.25 * (drm * vn + m.rho * dvn);
+  df[0] = 2.0 * dh;
+  for (int k = 0; k < DIM; ++k) df[k + 1] = dh * vs[k] + h * dvs[k] + dp * n[k];
+  df[DIM + 1] = dh * (inv_gm1 * m.B + dot) + h * (inv_gm1 * dB + ddot) + 0.5 * (dp * vn + m.p * dvn);
 }
 
-// abar += (df/dq_a)^T g, bbar += (df/dq_b)^T g.
+// abar += (df/dq_a)^T g, bbar += (df/dq_b)^T g (kin, which the flux does not
+// take, untouched).
 template <int DIM>
 DG_HD void chandrashekar_vjp(double inv_gm1, const NodePrims<DIM>& a, const NodePrims<DIM>& b,
                              const double* n, const double* g, PrimTangent<DIM>& abar,
                              PrimTangent<DIM>& bbar) {
   const ChandrashekarMeans m = chandrashekar_means<DIM>(a, b);
-  double vna = 0.0, vnb = 0.0;
-  for (int k = 0; k < DIM; ++k) {
-    vna += a.v[k] * n[k];
-    vnb += b.v[k] * n[k];
-  }
-  const double f1 = m.rho * 0.5 * (vna + vnb);
-  const double A = 0.5 * (inv_gm1 * m.B - (a.kin + b.kin));
   const double gE = g[DIM + 1];
-  double f1b = g[0] + gE * A;
-  double pmb = 0.0;
+  double vs[DIM], vn = 0.0, dot = 0.0, hb = 2.0 * g[0], pb = 0.0;
   for (int k = 0; k < DIM; ++k) {
-    const double vavg = 0.5 * (a.v[k] + b.v[k]);
-    const double fk = f1 * vavg + m.p * n[k];
-    const double gk = g[k + 1] + gE * vavg;  // cotangent of f_k (own and in f_E)
-    f1b += gk * vavg;
-    pmb += gk * n[k];
-    const double vavgb = gk * f1 + gE * fk;
-    abar.v[k] += 0.5 * vavgb;
-    bbar.v[k] += 0.5 * vavgb;
+    vs[k] = a.v[k] + b.v[k];
+    vn += vs[k] * n[k];
+    dot += a.v[k] * b.v[k];
+    hb += g[k + 1] * vs[k];
+    pb += g[k + 1] * n[k];
   }
-  const double Bb = gE * f1 * 0.5 * inv_gm1;
-  const double vsqb = -gE * f1 * 0.5;
-  const double rmb = f1b * 0.5 * (vna + vnb);
-  const double vnb_ = f1b * m.rho * 0.5;  // cotangent of vna and of vnb
+  const double h = 0.25 * m.rho * vn;
+  hb += gE * (inv_gm1 * m.B + dot);
+  pb += 0.5 * gE * vn;
+  const double vnb = 0.25 * m.rho * hb + 0.5 * gE * m.p, dotb = gE * h;
   for (int k = 0; k < DIM; ++k) {
-    abar.v[k] += vnb_ * n[k];
-    bbar.v[k] += vnb_ * n[k];
+    const double vsb = h * g[k + 1] + vnb * n[k];
+    abar.v[k] += vsb + dotb * b.v[k];
+    bbar.v[k] += vsb + dotb * a.v[k];
   }
-  abar.kin += vsqb;
-  bbar.kin += vsqb;
-  abar.rho += m.rho_a * rmb + m.p_rho * pmb;
-  bbar.rho += m.rho_b * rmb + m.p_rho * pmb;
-  abar.beta += m.B_a * Bb + m.p_beta * pmb;
-  bbar.beta += m.B_b * Bb + m.p_beta * pmb;
+  const double rmb = 0.25 * vn * hb, Bb = dotb * inv_gm1;
+  abar.rho += m.rho_a * rmb + m.p_rho * pb;
+  bbar.rho += m.rho_b * rmb + m.p_rho * pb;
+  abar.beta += m.B_a * Bb + m.p_beta * pb;
+  bbar.beta += m.B_b * Bb + m.p_beta * pb;
 }
 
 // ---------------------------------------------------------------------
@@ -205,7 +203,7 @@ DG_HD void chandrashekar_vjp(double inv_gm1, const NodePrims<DIM>& a, const Node
 // dp = (gamma - 1)(dE - v.dm + kin drho).
 template <int DIM>
 DG_HD void vp_jvp(double gamma, const NodePrims<DIM>& q, const double* du, double* dv, double& dp) {
-  const double ir = 1.0 / q.rho;
+  const double ir = recip(q.rho);
   double vdm = 0.0;
   for (int k = 0; k < DIM; ++k) {
     dv[k] = (du[k + 1] - q.v[k] * du[0]) * ir;
@@ -218,7 +216,7 @@ DG_HD void vp_jvp(double gamma, const NodePrims<DIM>& q, const double* du, doubl
 template <int DIM>
 DG_HD void vp_vjp(double gamma, const NodePrims<DIM>& q, const double* vbar, double pbar,
                   double* ubar) {
-  const double ir = 1.0 / q.rho;
+  const double ir = recip(q.rho);
   double rb = (gamma - 1.0) * q.kin * pbar;
   for (int k = 0; k < DIM; ++k) {
     ubar[k + 1] += vbar[k] * ir - (gamma - 1.0) * q.v[k] * pbar;
@@ -296,8 +294,8 @@ DG_HD void llf_lambda_grad(double gamma, const NodePrims<DIM>& ql, const NodePri
   if (wc != 0.0) {
     // c = sqrt(gamma p / rho): dc = c/2 (dp/p - drho/rho)
     const double w = wc * sqrt(nn) * 0.5 * q.c;
-    pb += w / q.p;
-    grad[0] -= w / q.rho;
+    pb += w * recip(q.p);
+    grad[0] -= w * recip(q.rho);
   }
   vp_vjp<DIM>(gamma, q, vb, pb, grad);
 }
@@ -378,8 +376,17 @@ DG_HD Dual operator-(Dual a, Dual b) { return Dual(a.v - b.v, a.d - b.d); }
 DG_HD Dual operator-(Dual a) { return Dual(-a.v, -a.d); }
 DG_HD Dual operator*(Dual a, Dual b) { return Dual(a.v * b.v, a.d * b.v + a.v * b.d); }
 DG_HD Dual operator/(Dual a, Dual b) {
-  const double q = a.v / b.v;
-  return Dual(q, (a.d - q * b.d) / b.v);
+  const double y = recip(b.v), q = div_by(a.v, b.v, y);
+  return Dual(q, (a.d - q * b.d) * y);
+}
+DG_HD Dual recip(Dual a) {
+  const double y = recip(a.v);
+  return Dual(y, -a.d * y * y);
+}
+// a / b with y = recip(b)
+DG_HD Dual div_by(Dual a, Dual b, Dual y) {
+  const double q = div_by(a.v, b.v, y.v);
+  return Dual(q, (a.d - q * b.d) * y.v);
 }
 DG_HD Dual sqrt(Dual a) {
   const double r = sqrt(a.v);
@@ -442,30 +449,32 @@ DG_HD void hllc_vjp(double gamma, const double* ul, const double* ur, const doub
   double nrm = 0.0, nh[DIM], vl[DIM], vr[DIM];
   for (int d = 0; d < DIM; ++d) nrm += n[d] * n[d];
   nrm = sqrt(nrm);
-  for (int d = 0; d < DIM; ++d) nh[d] = n[d] / nrm;
+  const double inrm = recip(nrm);
+  for (int d = 0; d < DIM; ++d) nh[d] = div_by(n[d], nrm, inrm);
   const double rl = ul[0], rr = ur[0], El = ul[NV - 1], Er = ur[NV - 1];
+  const double il = recip(rl), ir = recip(rr);
   double v2l = 0.0, v2r = 0.0, vnl = 0.0, vnr = 0.0;
   for (int d = 0; d < DIM; ++d) {
-    vl[d] = ul[d + 1] / rl;
-    vr[d] = ur[d + 1] / rr;
+    vl[d] = div_by(ul[d + 1], rl, il);
+    vr[d] = div_by(ur[d + 1], rr, ir);
     v2l += vl[d] * vl[d];
     v2r += vr[d] * vr[d];
     vnl += vl[d] * nh[d];
     vnr += vr[d] * nh[d];
   }
-  const double el = El / rl, er = Er / rr;
+  const double el = div_by(El, rl, il), er = div_by(Er, rr, ir);
   const double pl = (gamma - 1.0) * (El - 0.5 * rl * v2l);
   const double pr = (gamma - 1.0) * (Er - 0.5 * rr * v2r);
-  const double cl = sqrt(gamma * pl / rl), cr = sqrt(gamma * pr / rr);
-  const double sl = sqrt(rl), sr = sqrt(rr), ss = sl + sr;
+  const double cl = sqrt(div_by(gamma * pl, rl, il)), cr = sqrt(div_by(gamma * pr, rr, ir));
+  const double sl = sqrt(rl), sr = sqrt(rr), ss = sl + sr, is = recip(ss);
   double vd[DIM], vroe2 = 0.0;
   for (int d = 0; d < DIM; ++d) {
-    vd[d] = (sl * vl[d] + sr * vr[d]) / ss;
+    vd[d] = div_by(sl * vl[d] + sr * vr[d], ss, is);
     vroe2 += vd[d] * vd[d];
   }
-  const double vroe = (sl * vnl + sr * vnr) / ss;
-  const double Hl = (El + pl) / rl, Hr = (Er + pr) / rr;
-  const double Hroe = (sl * Hl + sr * Hr) / ss;
+  const double vroe = div_by(sl * vnl + sr * vnr, ss, is);
+  const double Hl = div_by(El + pl, rl, il), Hr = div_by(Er + pr, rr, ir);
+  const double Hroe = div_by(sl * Hl + sr * Hr, ss, is);
   const double croe = sqrt((gamma - 1.0) * (Hroe - 0.5 * vroe2));
   // SL = dmin(vnl - cl, vroe - croe), SR = dmax(vnr + cr, vroe + croe)
   const double aL = vnl - cl, bL = vroe - croe, aR = vnr + cr, bR = vroe + croe;
@@ -473,10 +482,11 @@ DG_HD void hllc_vjp(double gamma, const double* ul, const double* ur, const doub
   const double SL = SL_roe ? bL : aL, SR = SR_roe ? bR : aR;
   const double mL = SL - vnl, mR = SR - vnr;
   const bool star = !(SL >= 0) && !(SR <= 0);
-  double Ss = 0.0, Den = 1.0;
+  double Ss = 0.0, iden = 1.0;
   if (star) {
-    Den = rl * mL - rr * mR;
-    Ss = (pr - pl + rl * vnl * mL - rr * vnr * mR) / (rl * mL - rr * mR);
+    const double den = rl * mL - rr * mR;
+    iden = recip(den);
+    Ss = div_by(pr - pl + rl * vnl * mL - rr * vnr * mR, den, iden);
   }
   const bool left = star ? Ss >= 0 : SL >= 0;
   const double* uk = left ? ul : ur;
@@ -494,8 +504,8 @@ DG_HD void hllc_vjp(double gamma, const double* ul, const double* ur, const doub
     const double* vk = left ? vl : vr;
     const double rk = left ? rl : rr, vnk = left ? vnl : vnr, ek = left ? el : er;
     const double pk = left ? pl : pr, Sk = left ? SL : SR, mk = left ? mL : mR;
-    const double D = Sk - Ss, rs = rk * mk / D;
-    const double X = Ss - vnk, rkmk = rk * mk, Z = pk / rkmk, Y = Ss + Z, es = ek + X * Y;
+    const double iD = recip(Sk - Ss), rs = rk * mk * iD;
+    const double X = Ss - vnk, irkmk = recip(rk * mk), Z = pk * irkmk, Y = Ss + Z, es = ek + X * Y;
     // f0 = fk0 + Sk (rs - uk0), f_d = fk_d + Sk (rs (vk_d + X nh_d) - uk_d),
     // fE = fkE + Sk (rs es - ukE)
     double Sk_b = G[0] * (rs - uk[0]) + G[NV - 1] * (rs * es - uk[NV - 1]);
@@ -513,14 +523,14 @@ DG_HD void hllc_vjp(double gamma, const double* ul, const double* ur, const doub
     const double Y_b = es_b * X, ek_b = es_b;
     // Y = Ss + pk / (rk mk)
     Ss_b += Y_b;
-    const double pk_b = Y_b / rkmk, rkmk_b = -Y_b * Z / rkmk;
+    const double pk_b = Y_b * irkmk, rkmk_b = -Y_b * Z * irkmk;
     // X = Ss - vnk
     Ss_b += X_b;
     double vnk_b = -X_b;
     // rs = rk mk / (Sk - Ss)
-    const double rk_b = rs_b * mk / D + rkmk_b * mk;
-    double mk_b = rs_b * rk / D + rkmk_b * rk;
-    const double D_b = -rs_b * rs / D;
+    const double rk_b = rs_b * mk * iD + rkmk_b * mk;
+    double mk_b = rs_b * rk * iD + rkmk_b * rk;
+    const double D_b = -rs_b * rs * iD;
     Sk_b += D_b;
     Ss_b -= D_b;
     double SL_b = 0.0, SR_b = 0.0, mL_b = 0.0, mR_b = 0.0;
@@ -532,7 +542,7 @@ DG_HD void hllc_vjp(double gamma, const double* ul, const double* ur, const doub
       for (int d = 0; d < DIM; ++d) vr_b[d] += vk_b[d];
     }
     // Ss = (pr - pl + rl vnl mL - rr vnr mR) / (rl mL - rr mR)
-    const double Num_b = Ss_b / Den, Den_b = -Ss_b * Ss / Den;
+    const double Num_b = Ss_b * iden, Den_b = -Ss_b * Ss * iden;
     pr_b += Num_b;
     pl_b -= Num_b;
     rl_b += Num_b * vnl * mL + Den_b * mL;
@@ -563,53 +573,53 @@ DG_HD void hllc_vjp(double gamma, const double* ul, const double* ur, const doub
       cr_b += SR_b;
     }
     // croe = sqrt((gamma - 1)(Hroe - vroe2 / 2))
-    const double W_b = croe_b / (2.0 * croe);
+    const double W_b = croe_b * recip(2.0 * croe);
     const double Hroe_b = gm1 * W_b, vroe2_b = -0.5 * gm1 * W_b;
-    double sl_b = Hroe_b * (Hl - Hroe) / ss + vroe_b * (vnl - vroe) / ss;
-    double sr_b = Hroe_b * (Hr - Hroe) / ss + vroe_b * (vnr - vroe) / ss;
-    const double Hl_b = Hroe_b * sl / ss, Hr_b = Hroe_b * sr / ss;
-    vnl_b += vroe_b * sl / ss;
-    vnr_b += vroe_b * sr / ss;
+    double sl_b = Hroe_b * (Hl - Hroe) * is + vroe_b * (vnl - vroe) * is;
+    double sr_b = Hroe_b * (Hr - Hroe) * is + vroe_b * (vnr - vroe) * is;
+    const double Hl_b = Hroe_b * sl * is, Hr_b = Hroe_b * sr * is;
+    vnl_b += vroe_b * sl * is;
+    vnr_b += vroe_b * sr * is;
     for (int d = 0; d < DIM; ++d) {
       const double vd_b = 2.0 * vd[d] * vroe2_b;
-      vl_b[d] += vd_b * sl / ss;
-      vr_b[d] += vd_b * sr / ss;
-      sl_b += vd_b * (vl[d] - vd[d]) / ss;
-      sr_b += vd_b * (vr[d] - vd[d]) / ss;
+      vl_b[d] += vd_b * sl * is;
+      vr_b[d] += vd_b * sr * is;
+      sl_b += vd_b * (vl[d] - vd[d]) * is;
+      sr_b += vd_b * (vr[d] - vd[d]) * is;
     }
     // H = (E + p) / rho, s = sqrt(rho), c = sqrt(gamma p / rho)
-    El_b += Hl_b / rl;
-    pl_b += Hl_b / rl;
-    rl_b -= Hl_b * Hl / rl;
-    Er_b += Hr_b / rr;
-    pr_b += Hr_b / rr;
-    rr_b -= Hr_b * Hr / rr;
-    rl_b += sl_b / (2.0 * sl);
-    rr_b += sr_b / (2.0 * sr);
+    El_b += Hl_b * il;
+    pl_b += Hl_b * il;
+    rl_b -= Hl_b * Hl * il;
+    Er_b += Hr_b * ir;
+    pr_b += Hr_b * ir;
+    rr_b -= Hr_b * Hr * ir;
+    rl_b += sl_b * recip(2.0 * sl);
+    rr_b += sr_b * recip(2.0 * sr);
     if (cl_b != 0.0) {
-      const double Q_b = cl_b / (2.0 * cl);
-      pl_b += Q_b * gamma / rl;
-      rl_b -= Q_b * cl * cl / rl;
+      const double Q_b = cl_b * recip(2.0 * cl);
+      pl_b += Q_b * gamma * il;
+      rl_b -= Q_b * cl * cl * il;
     }
     if (cr_b != 0.0) {
-      const double Q_b = cr_b / (2.0 * cr);
-      pr_b += Q_b * gamma / rr;
-      rr_b -= Q_b * cr * cr / rr;
+      const double Q_b = cr_b * recip(2.0 * cr);
+      pr_b += Q_b * gamma * ir;
+      rr_b -= Q_b * cr * cr * ir;
     }
   }
   // e = E / rho, p = (gamma - 1)(E - rho |v|^2 / 2), v = m / rho
-  El_b += el_b / rl + gm1 * pl_b;
-  rl_b -= el_b * el / rl + 0.5 * gm1 * v2l * pl_b;
-  Er_b += er_b / rr + gm1 * pr_b;
-  rr_b -= er_b * er / rr + 0.5 * gm1 * v2r * pr_b;
+  El_b += el_b * il + gm1 * pl_b;
+  rl_b -= el_b * el * il + 0.5 * gm1 * v2l * pl_b;
+  Er_b += er_b * ir + gm1 * pr_b;
+  rr_b -= er_b * er * ir + 0.5 * gm1 * v2r * pr_b;
   const double v2l_b = -0.5 * gm1 * rl * pl_b, v2r_b = -0.5 * gm1 * rr * pr_b;
   for (int d = 0; d < DIM; ++d) {
     vl_b[d] += 2.0 * vl[d] * v2l_b + vnl_b * nh[d];
     vr_b[d] += 2.0 * vr[d] * v2r_b + vnr_b * nh[d];
-    ulb[d + 1] += vl_b[d] / rl;
-    rl_b -= vl_b[d] * vl[d] / rl;
-    urb[d + 1] += vr_b[d] / rr;
-    rr_b -= vr_b[d] * vr[d] / rr;
+    ulb[d + 1] += vl_b[d] * il;
+    rl_b -= vl_b[d] * vl[d] * il;
+    urb[d + 1] += vr_b[d] * ir;
+    rr_b -= vr_b[d] * vr[d] * ir;
   }
   ulb[0] += rl_b;
   ulb[NV - 1] += El_b;
@@ -630,7 +640,7 @@ DG_HD void hllc_vjp(double gamma, const double* ul, const double* ur, const doub
 
 template <int DIM>
 DG_HD void grad_vars_jvp(double gamma, const double* u, const double* du, double* dq) {
-  const double ir = 1.0 / u[0];
+  const double ir = recip(u[0]);
   double m2 = 0.0, mdm = 0.0;
   for (int k = 0; k < DIM; ++k) {
     m2 += u[k + 1] * u[k + 1];
@@ -645,7 +655,7 @@ DG_HD void grad_vars_jvp(double gamma, const double* u, const double* du, double
 
 template <int DIM>
 DG_HD void grad_vars_vjp(double gamma, const double* u, const double* qbar, double* ubar) {
-  const double ir = 1.0 / u[0];
+  const double ir = recip(u[0]);
   double m2 = 0.0;
   for (int k = 0; k < DIM; ++k) m2 += u[k + 1] * u[k + 1];
   const double p = (gamma - 1.0) * (u[DIM + 1] - 0.5 * m2 * ir);
@@ -663,18 +673,20 @@ DG_HD void grad_vars_vjp(double gamma, const double* u, const double* qbar, doub
   ubar[0] += rb;
 }
 
+DG_HD double third(double x) { return div_by(x, 3.0, 1.0 / 3.0); }
+
 // Symmetric viscous stress tau (without mu) from the velocity gradients
 // g[c][1 + k] = d v_k / d x_c, as viscous_flux_dir forms it.
 template <int DIM>
 DG_HD void stress(const double g[DIM][DIM + 2], double tau[DIM][DIM]) {
   if constexpr (DIM == 2) {
-    tau[0][0] = (4.0 * g[0][1] - 2.0 * g[1][2]) / 3.0;
-    tau[1][1] = (4.0 * g[1][2] - 2.0 * g[0][1]) / 3.0;
+    tau[0][0] = third(4.0 * g[0][1] - 2.0 * g[1][2]);
+    tau[1][1] = third(4.0 * g[1][2] - 2.0 * g[0][1]);
     tau[0][1] = tau[1][0] = g[1][1] + g[0][2];
   } else {
-    tau[0][0] = (4.0 * g[0][1] - 2.0 * (g[1][2] + g[2][3])) / 3.0;
-    tau[1][1] = (4.0 * g[1][2] - 2.0 * (g[0][1] + g[2][3])) / 3.0;
-    tau[2][2] = (4.0 * g[2][3] - 2.0 * (g[0][1] + g[1][2])) / 3.0;
+    tau[0][0] = third(4.0 * g[0][1] - 2.0 * (g[1][2] + g[2][3]));
+    tau[1][1] = third(4.0 * g[1][2] - 2.0 * (g[0][1] + g[2][3]));
+    tau[2][2] = third(4.0 * g[2][3] - 2.0 * (g[0][1] + g[1][2]));
     tau[0][1] = tau[1][0] = g[1][1] + g[0][2];
     tau[0][2] = tau[2][0] = g[2][1] + g[0][3];
     tau[1][2] = tau[2][1] = g[2][2] + g[1][3];
@@ -687,8 +699,8 @@ template <int DIM>
 DG_HD void stress_vjp(const double taubar[DIM][DIM], double gbar[DIM][DIM + 2]) {
   if constexpr (DIM == 2) {
     const double t00 = taubar[0][0], t11 = taubar[1][1], t01 = taubar[0][1] + taubar[1][0];
-    gbar[0][1] += (4.0 * t00 - 2.0 * t11) / 3.0;
-    gbar[1][2] += (4.0 * t11 - 2.0 * t00) / 3.0;
+    gbar[0][1] += third(4.0 * t00 - 2.0 * t11);
+    gbar[1][2] += third(4.0 * t11 - 2.0 * t00);
     gbar[1][1] += t01;
     gbar[0][2] += t01;
   } else {
@@ -696,9 +708,9 @@ DG_HD void stress_vjp(const double taubar[DIM][DIM], double gbar[DIM][DIM + 2]) 
     const double t01 = taubar[0][1] + taubar[1][0];
     const double t02 = taubar[0][2] + taubar[2][0];
     const double t12 = taubar[1][2] + taubar[2][1];
-    gbar[0][1] += (4.0 * t00 - 2.0 * (t11 + t22)) / 3.0;
-    gbar[1][2] += (4.0 * t11 - 2.0 * (t00 + t22)) / 3.0;
-    gbar[2][3] += (4.0 * t22 - 2.0 * (t00 + t11)) / 3.0;
+    gbar[0][1] += third(4.0 * t00 - 2.0 * (t11 + t22));
+    gbar[1][2] += third(4.0 * t11 - 2.0 * (t00 + t22));
+    gbar[2][3] += third(4.0 * t22 - 2.0 * (t00 + t11));
     gbar[1][1] += t01;
     gbar[0][2] += t01;
     gbar[2][1] += t02;
@@ -709,13 +721,12 @@ DG_HD void stress_vjp(const double taubar[DIM][DIM], double gbar[DIM][DIM + 2]) 
 }
 
 // Tangent of the viscous flux in every direction c: f[c] = (0, mu tau[c][.],
-// mu (v . tau[c][.] + kappa dT/dx_c)).
+// mu (v . tau[c][.] + kappa dT/dx_c)), tau the stress of the gradient.
 template <int DIM>
-DG_HD void viscous_flux_jvp(double mu, double kappa, const double* q, const double g[DIM][DIM + 2],
-                            const double* dq, const double dg[DIM][DIM + 2],
-                            double df[DIM][DIM + 2]) {
-  double tau[DIM][DIM], dtau[DIM][DIM];
-  stress<DIM>(g, tau);
+DG_HD void viscous_flux_jvp_stress(double mu, double kappa, const double* q,
+                                   const double tau[DIM][DIM], const double* dq,
+                                   const double dg[DIM][DIM + 2], double df[DIM][DIM + 2]) {
+  double dtau[DIM][DIM];
   stress<DIM>(dg, dtau);
   for (int c = 0; c < DIM; ++c) {
     df[c][0] = 0.0;
@@ -728,13 +739,21 @@ DG_HD void viscous_flux_jvp(double mu, double kappa, const double* q, const doub
   }
 }
 
+template <int DIM>
+DG_HD void viscous_flux_jvp(double mu, double kappa, const double* q, const double g[DIM][DIM + 2],
+                            const double* dq, const double dg[DIM][DIM + 2],
+                            double df[DIM][DIM + 2]) {
+  double tau[DIM][DIM];
+  stress<DIM>(g, tau);
+  viscous_flux_jvp_stress<DIM>(mu, kappa, q, tau, dq, dg, df);
+}
+
 // qbar += (df/dq)^T fbar, gbar += (df/dg)^T fbar over all directions c.
 template <int DIM>
-DG_HD void viscous_flux_vjp(double mu, double kappa, const double* q, const double g[DIM][DIM + 2],
-                            const double fbar[DIM][DIM + 2], double* qbar,
-                            double gbar[DIM][DIM + 2]) {
-  double tau[DIM][DIM], taubar[DIM][DIM];
-  stress<DIM>(g, tau);
+DG_HD void viscous_flux_vjp_stress(double mu, double kappa, const double* q,
+                                   const double tau[DIM][DIM], const double fbar[DIM][DIM + 2],
+                                   double* qbar, double gbar[DIM][DIM + 2]) {
+  double taubar[DIM][DIM];
   for (int c = 0; c < DIM; ++c) {
     const double fe = mu * fbar[c][DIM + 1];
     gbar[c][DIM + 1] += kappa * fe;
@@ -744,6 +763,15 @@ DG_HD void viscous_flux_vjp(double mu, double kappa, const double* q, const doub
     }
   }
   stress_vjp<DIM>(taubar, gbar);
+}
+
+template <int DIM>
+DG_HD void viscous_flux_vjp(double mu, double kappa, const double* q, const double g[DIM][DIM + 2],
+                            const double fbar[DIM][DIM + 2], double* qbar,
+                            double gbar[DIM][DIM + 2]) {
+  double tau[DIM][DIM];
+  stress<DIM>(g, tau);
+  viscous_flux_vjp_stress<DIM>(mu, kappa, q, tau, fbar, qbar, gbar);
 }
 
 }  // namespace dgsem
