@@ -63,7 +63,7 @@ void release(dgsem_handle* h) {
   hipFree(h->d_invJ);
   hipFree(h->d_sn);
   hipFree(h->d_nbr);
-  hipFree(h->d_Vinv);
+  hipFree(h->d_basis);
   hipFree(h->d_ja_box);
   hipFree(h->d_alpha);
   hipFree(h->d_visc);
@@ -78,7 +78,7 @@ void release(dgsem_handle* h) {
   hipFree(h->d_fl_w);
   h->d_ad_dgrad = h->d_ad_qbar = h->d_wq = h->d_ke_partial = nullptr;
   h->d_an_partial = h->d_ad_alpha = h->d_ad_out = h->d_fl_r = h->d_fl_w = nullptr;
-  h->d_Ja = h->d_invJ = h->d_sn = h->d_Vinv = h->d_alpha = h->d_visc = nullptr;
+  h->d_Ja = h->d_invJ = h->d_sn = h->d_basis = h->d_alpha = h->d_visc = nullptr;
   h->d_nbr = nullptr;
   h->d_ja_box = nullptr;
 }
@@ -145,6 +145,14 @@ std::vector<int> neighbour_table(const dgsem::Geometry& g, const int* periodic) 
   return nb;
 }
 
+// The table of dgsem::Operators.
+std::vector<double> basis_operators(const dgsem::BasisTables& b) {
+  std::vector<double> t;
+  for (const std::vector<double>* v : {&b.Dsplit, &b.Dhat, &b.Vinv, &b.inv_weights})
+    t.insert(t.end(), v->begin(), v->end());
+  return t;
+}
+
 void fill_params(dgsem_handle* h) {
   dgsem::KParams& p = h->base;
   const auto& c = h->cfg;
@@ -154,7 +162,7 @@ void fill_params(dgsem_handle* h) {
   p.invJ = h->d_invJ;
   p.sn = h->d_sn;
   p.nbr = h->d_nbr;
-  p.Vinv = h->d_Vinv;
+  p.basis = h->d_basis;
   p.alpha = h->d_alpha;
   p.alpha_in = nullptr;
   p.ja_box = h->d_ja_box;
@@ -176,13 +184,6 @@ void fill_params(dgsem_handle* h) {
   p.floor_value = c.positivity_floor;
   p.lhat0 = b.lhat_left[0];
   p.lhatN = b.lhat_right[b.n - 1];
-  for (int i = 0; i < b.n; ++i) {
-    p.inv_w[i] = b.inv_weights[i];
-    for (int j = 0; j < b.n; ++j) {
-      p.Ds[i][j] = b.Dsplit[i * b.n + j];
-      p.Dhat[i][j] = b.Dhat[i * b.n + j];
-    }
-  }
   // Navier-Stokes: kappa = gamma / ((gamma - 1) Pr), compressible_navier_stokes3D.hpp:19-22
   p.mu = c.mu;
   p.kappa = c.gamma / ((c.gamma - 1.0) * c.prandtl);
@@ -400,7 +401,7 @@ int dgsem_create(const dgsem_config* cfg, void* stream, dgsem_handle** out) {
     sn = h->geo.subcell_normals;
   if ((rc = upload(h, &h->d_Ja, Ja)) || (rc = upload(h, &h->d_invJ, invJ)) ||
       (rc = upload(h, &h->d_sn, sn)) || (rc = upload(h, &h->d_nbr, neighbour_table(h->geo, periodic))) ||
-      (rc = upload(h, &h->d_Vinv, h->basis.Vinv)) ||
+      (rc = upload(h, &h->d_basis, basis_operators(h->basis))) ||
       (rc = upload(h, &h->d_alpha, std::vector<double>(4 * h->E, 0.0))) ||
       (h->cfg.equation == DGSEM_NAVIER_STOKES &&
        (rc = alloc_zero(h, &h->d_visc, (size_t)h->E * h->cfg.dim * h->nvars * h->nn)))) {

@@ -197,6 +197,14 @@ int ad_prepare(dgsem_handle* h) {
 
 dgsem::AdParams ad_params(dgsem_handle* h, const double* u) {
   dgsem::AdParams a{};
+  const dgsem::BasisTables& b = h->basis;
+  for (int i = 0; i < b.n; ++i) {
+    a.inv_w[i] = b.inv_weights[i];
+    for (int j = 0; j < b.n; ++j) {
+      a.Ds[i][j] = b.Dsplit[i * b.n + j];
+      a.Dhat[i][j] = b.Dhat[i * b.n + j];
+    }
+  }
   a.k = h->base;
   a.k.u = u;
   a.dgrad = h->cfg.equation == DGSEM_NAVIER_STOKES ? h->d_ad_dgrad : nullptr;

@@ -55,6 +55,16 @@ __device__ __forceinline__ double combine(const AdParams& a, int64_t g, double r
   return o;
 }
 
+// The basis operators among the kernel's arguments.  The derivative kernels use
+// them right after their first loads, where the table of Operators would put its
+// pointer's load in front (1.5% of a tangent plus adjoint at 16^3, N = 3).
+struct AdOperators {
+  const AdParams& a;
+  __device__ __forceinline__ double Ds(int i, int j) const { return a.Ds[i][j]; }
+  __device__ __forceinline__ double Dhat(int i, int j) const { return a.Dhat[i][j]; }
+  __device__ __forceinline__ double inv_w(int i) const { return a.inv_w[i]; }
+};
+
 template <int DIM, int NN>
 __device__ __forceinline__ void load_state(const double* u, int64_t e, int node, double* s) {
   for (int v = 0; v < DIM + 2; ++v) s[v] = u[(e * (DIM + 2) + v) * NN + node];
@@ -308,6 +318,7 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) jvp_viscous_kern
   constexpr int SG = DIM * ND * PN + S::slot_pad(DIM * ND * PN);
   static_assert(DIM >= 2, "q and dq fit the planes of the line derivatives");
   const KParams& p = a.k;
+  const AdOperators op{a};
   __shared__ double s_g[EPW * SG];  // q and dq [var], then the derivatives [dir][var]
   const int tid = threadIdx.x;
   const int64_t e0 = (int64_t)xcd_block(blockIdx.x, gridDim.x) * EPW;
@@ -362,8 +373,8 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) jvp_viscous_kern
     for (int k = 0; k < n; ++k)
 #pragma unroll
       for (int v = 0; v < ND; ++v) x[k][v] = s_g[l.slot * SG + v * PN + l.pos(k)];
-    line_gradient<DIM, N, NODAL, DIM == 2>(p, l.e, l.eid, l.dir, l.line, l.first(), l.last(), x, q_lo,
-                                           q_hi, l.blo, l.bhi, sg_lo, sg_hi, acc);
+    line_gradient<DIM, N, NODAL, DIM == 2>(p, op, l.e, l.eid, l.dir, l.line, l.first(), l.last(), x,
+                                           q_lo, q_hi, l.blo, l.bhi, sg_lo, sg_hi, acc);
     double dx[n][ND];
 #pragma unroll
     for (int k = 0; k < n; ++k)
@@ -375,7 +386,7 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) jvp_viscous_kern
       for (int v = 0; v < ND; ++v) {
         double r = 0.0;
 #pragma unroll
-        for (int i = 0; i < n; ++i) r += p.Dhat[k][i] * dx[i][v];
+        for (int i = 0; i < n; ++i) r += op.Dhat(k, i) * dx[i][v];
         dacc[k][v] = r;
       }
 #pragma unroll
@@ -472,6 +483,7 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES))
   constexpr int BLOCK = EPW * S::LINES, NODES = EPW * NN, PASSES = (NODES + BLOCK - 1) / BLOCK;
   constexpr int SQ = NQ * PN + S::slot_pad(NQ * PN);
   const KParams& p = a.k;
+  const AdOperators op{a};
   __shared__ double s_p[EPW * SQ];   // rho, v, beta; later the per-direction sums
   __shared__ double s_dq[EPW * SQ];  // their tangents
   double* const s_acc = s_p;
@@ -612,7 +624,7 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES))
 #pragma unroll
         for (int c = 0; c < DIM; ++c) nrm[c] = NODAL ? ja[NODAL ? ia : 0][c] + ja[NODAL ? ib : 0][c] : ja[0][c];
         chandrashekar_jvp<DIM>(p.inv_gm1, qa, qb, ta, tb, nrm, df);
-        const double wa = coef * p.Ds[ia][ib], wb = coef * p.Ds[ib][ia];
+        const double wa = coef * op.Ds(ia, ib), wb = coef * op.Ds(ib, ia);
 #pragma unroll
         for (int v = 0; v < NV; ++v) {
           acc[ia][v] += wa * df[v];
@@ -644,7 +656,7 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES))
           else
             llf_jvp<DIM>(p.gamma, ul, node_prims<DIM>(p.gamma, ul), ur, node_prims<DIM>(p.gamma, ur),
                          dul, dur, nrm, df);
-          const double wl = alpha * p.inv_w[fi - 1], wr = alpha * p.inv_w[fi];
+          const double wl = alpha * op.inv_w(fi - 1), wr = alpha * op.inv_w(fi);
           for (int v = 0; v < NV; ++v) {
             acc[fi - 1][v] += wl * df[v];
             acc[fi][v] -= wr * df[v];
@@ -680,7 +692,7 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES))
         for (int k = 0; k < n; ++k) {
           double r = 0.0;
 #pragma unroll
-          for (int i = 0; i < n; ++i) r += p.Dhat[k][i] * x[i];
+          for (int i = 0; i < n; ++i) r += op.Dhat(k, i) * x[i];
           if (k == 0 && v < lo_end) r -= sg_lo * x[0] * p.lhat0;
           if (k == n - 1 && v < hi_end) r += sg_hi * up * p.lhatN;
           acc[k][v] += r;
@@ -737,6 +749,7 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) vjp_viscous_kern
   constexpr int BLOCK = EPW * S::LINES, NODES = EPW * NN, PASSES = (NODES + BLOCK - 1) / BLOCK;
   constexpr int SG = DIM * ND * PN + S::slot_pad(DIM * ND * PN);
   const KParams& p = a.k;
+  const AdOperators op{a};
   __shared__ double s_g[EPW * SG];  // q and r [var], then G and Hbar [dir][var]
   const int tid = threadIdx.x;
   const int64_t e0 = (int64_t)xcd_block(blockIdx.x, gridDim.x) * EPW;
@@ -784,8 +797,8 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) vjp_viscous_kern
     for (int k = 0; k < n; ++k)
 #pragma unroll
       for (int v = 0; v < ND; ++v) x[k][v] = s_g[l.slot * SG + v * PN + l.pos(k)];
-    line_gradient<DIM, N, NODAL, DIM == 2>(p, l.e, l.eid, l.dir, l.line, l.first(), l.last(), x, q_lo,
-                                           q_hi, l.blo, l.bhi, sg_lo, sg_hi, acc);
+    line_gradient<DIM, N, NODAL, DIM == 2>(p, op, l.e, l.eid, l.dir, l.line, l.first(), l.last(), x,
+                                           q_lo, q_hi, l.blo, l.bhi, sg_lo, sg_hi, acc);
     double rx[n][ND];
 #pragma unroll
     for (int k = 0; k < n; ++k)
@@ -798,7 +811,7 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) vjp_viscous_kern
       for (int v = 0; v < ND; ++v) {
         double h = 0.0;
 #pragma unroll
-        for (int i = 0; i < n; ++i) h += p.Dhat[i][k] * rx[i][v];
+        for (int i = 0; i < n; ++i) h += op.Dhat(i, k) * rx[i][v];
         hb[k][v] = h;
       }
     // the first node's value is lifted by this element (-l_hat0, lower face)
@@ -922,6 +935,7 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES))
   constexpr int SQ = NQ * PN + S::slot_pad(NQ * PN), SU = S::SU;
   constexpr int SD = NS ? ND * PN + S::slot_pad(ND * PN) : 0;
   const KParams& p = a.k;
+  const AdOperators op{a};
   __shared__ double s_p[EPW * SQ];  // rho, v, beta; later their cotangents' sums
   __shared__ double s_r[EPW * SU];
   // conservative cotangents of the faces and subcells; without the subcells'
@@ -1111,7 +1125,7 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES))
         double nrm[DIM], g[NV];
 #pragma unroll
         for (int c = 0; c < DIM; ++c) nrm[c] = NODAL ? ja[NODAL ? ia : 0][c] + ja[NODAL ? ib : 0][c] : ja[0][c];
-        const double wa = coef * p.Ds[ia][ib], wb = coef * p.Ds[ib][ia];
+        const double wa = coef * op.Ds(ia, ib), wb = coef * op.Ds(ib, ia);
 #pragma unroll
         for (int v = 0; v < NV; ++v) g[v] = wa * rr[v * PN + l.pos(ia)] + wb * rr[v * PN + l.pos(ib)];
         PrimTangent<DIM> xa{}, xb{};
@@ -1141,7 +1155,7 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES))
         for (int k = 0; k < n; ++k) {
           double h = 0.0;
 #pragma unroll
-          for (int i = 0; i < n; ++i) h += p.Dhat[i][k] * x[i];
+          for (int i = 0; i < n; ++i) h += op.Dhat(i, k) * x[i];
           qv[k][v - 1] = h;
         }
         x_lo[v] = -sg_lo * p.lhat0 * x[0];
@@ -1202,7 +1216,7 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES))
             load_state<DIM, NN>(p.u, l.e, l.dof(fi - 1), ul);
             load_state<DIM, NN>(p.u, l.e, l.dof(fi), ur);
             subcell_normal<DIM, N, NODAL>(p, l.e, l.dir, l.line, fi - 1, nrm);
-            const double wl = alpha * p.inv_w[fi - 1], wr = alpha * p.inv_w[fi];
+            const double wl = alpha * op.inv_w(fi - 1), wr = alpha * op.inv_w(fi);
             for (int v = 0; v < NV; ++v) {
               g[v] = wl * rr[v * PN + l.pos(fi - 1)] - wr * rr[v * PN + l.pos(fi)];
               ubl[v] = ubr[v] = 0.0;
@@ -1238,7 +1252,7 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES))
         load_state<DIM, NN>(p.u, l.e, l.dof(fi - 1), ul);
         load_state<DIM, NN>(p.u, l.e, l.dof(fi), ur);
         subcell_normal<DIM, N, NODAL>(p, l.e, l.dir, l.line, fi - 1, nrm);
-        const double wl = alpha * p.inv_w[fi - 1], wr = alpha * p.inv_w[fi];
+        const double wl = alpha * op.inv_w(fi - 1), wr = alpha * op.inv_w(fi);
         for (int v = 0; v < NV; ++v) {
           g[v] = wl * rr[v * PN + l.pos(fi - 1)] - wr * rr[v * PN + l.pos(fi)];
           ubl[v] = ubr[v] = 0.0;

@@ -23,7 +23,7 @@ struct dgsem_handle {
   double* d_invJ = nullptr;
   double* d_sn = nullptr;
   int* d_nbr = nullptr;
-  double* d_Vinv = nullptr;
+  double* d_basis = nullptr;  // basis operators (kernels.hpp, Operators)
   double* d_ja_box = nullptr;  // box-mesh table of the metric terms (KParams::ja_box)
   int64_t ja_box_off[3] = {0, 0, 0};
   double* d_alpha = nullptr;  // blending factor per element, [4][E]: slot 0 the last

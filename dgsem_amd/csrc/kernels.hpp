@@ -55,13 +55,15 @@ struct FastDiv {
   }
 };
 
+// Ordered by use: what a kernel's first loads need comes first, so that it
+// arrives with the first scalar load.
 struct KParams {
   const double* u;       // stage input, [E][NV][NN]
-  const double* u_base;  // base state for kModeStage3
-  double* out;           // L(u) or the stage result
-  double* alpha;         // [E] blending factor (shock capturing), written
-  const double* alpha_in;  // [E] frozen blending factor to use instead of the
-                           // indicator's (shock capturing), or null
+  const double* basis;   // operators of the 1D basis (Operators below)
+  int64_t E;
+  int cells[3];
+  int mode;
+  FastDiv div_y, div_z;  // by cells[1] and cells[2]
   // Box meshes (the linear mapping of a Cartesian box, nodal geometry): the
   // halved metric terms Ja^r_c / 2 of a node depend on its element only through the
   // element's indices in the directions other than c, so each distinct row
@@ -74,32 +76,54 @@ struct KParams {
   int64_t ja_box_off[3];
   const double* Ja;      // nodal: [E][dim][dim][NN]; affine: [E][dim][dim]
   const double* invJ;    // nodal: [E][NN]; affine: [E]
-  const double* sn;      // nodal subcell normals [E][dim][FN][N][dim]
-  const int* nbr;        // [E][2*dim] (lower, upper) neighbour per direction
-  const double* Vinv;    // [n][n] inverse Legendre Vandermonde
+  double gamma, inv_gm1;
+  double lhat0, lhatN;
   const double* visc;    // Navier-Stokes: viscous fluxes (parabolic_impl.hpp)
   double* visc_out;      // written by the viscous kernel
-  int64_t E;
-  int mode;
+  double mu, kappa;      // viscosity and gamma / ((gamma - 1) Pr)
+  const double* sn;      // nodal subcell normals [E][dim][FN][N][dim]
+  const double* alpha_in;  // [E] frozen blending factor to use instead of the
+                           // indicator's (shock capturing), or null
+  double* alpha;         // [E] blending factor (shock capturing), written
+  double alpha_max, alpha_min, atol, threshold, sfac;
   int surface_flux, fv_flux;  // FluxKind
   int volume_flux;            // VolumeFluxKind (read by the run-time flux kernels only)
+  const double* u_base;  // base state for kModeStage3
+  double* out;           // L(u) or the stage result
   double c1, c2, c3;
-  double gamma, inv_gm1;
-  double alpha_max, alpha_min, atol, threshold, sfac;
   double floor_value;
-  double lhat0, lhatN;
-  double mu, kappa;  // viscosity and gamma / ((gamma - 1) Pr)
-  double Ds[kMaxN1][kMaxN1];
-  double Dhat[kMaxN1][kMaxN1];
-  double inv_w[kMaxN1];
-  // boundary conditions (2D): element grid, kind per face (-x, +x, -y, +y;
-  // 0 = periodic, then nbr holds -1 at that face), constant Dirichlet states
-  // and optional per-node Dirichlet states
-  int cells[3];
-  FastDiv div_y, div_z;  // by cells[1] and cells[2]
+  const int* nbr;        // [E][2*dim] (lower, upper) neighbour per direction
+  // boundary conditions (2D): kind per face (-x, +x, -y, +y; 0 = periodic, then
+  // nbr holds -1 at that face), constant Dirichlet states and optional per-node
+  // Dirichlet states
   int bc[6];
   double bc_state[6][5];
   const double* bc_values[6];
+};
+
+// The basis operators of N + 1 = n nodes at KParams::basis: D_split, D_hat and
+// the inverse Legendre Vandermonde matrix, n x n each, then the n inverse
+// weights.  They sit in device memory rather than among the kernel's arguments:
+// a launch's arguments are new to every cache, the table is not (a kernel that
+// only sums 52 of 208 values takes 5.0 us a launch from arguments, 2.5 from a
+// table).  The table is constant while kernels run, so its loads are scalar
+// (address space 4).  One MI355X, with the arguments in the order of their use:
+// Sedov blast 32^3, N = 3, 313 -> 293 us a step; 2D Riemann problem 101 x 97,
+// N = 5, 261 -> 255 us for four; an ensemble of 64 2D cases 425 -> 404 us for two.
+template <int N>
+struct Operators {
+  static constexpr int n = N + 1;
+#if defined(__HIP_DEVICE_COMPILE__)
+  using Table = const __attribute__((address_space(4))) double*;
+#else
+  using Table = const double*;
+#endif
+  Table t;
+  __host__ __device__ explicit Operators(const KParams& p) : t((Table)p.basis) {}
+  __host__ __device__ double Ds(int i, int j) const { return t[i * n + j]; }
+  __host__ __device__ double Dhat(int i, int j) const { return t[n * n + i * n + j]; }
+  __host__ __device__ double Vinv(int i, int j) const { return t[2 * n * n + i * n + j]; }
+  __host__ __device__ double inv_w(int i) const { return t[3 * n * n + i]; }
 };
 
 // Per-(dim, N) launchers, explicitly specialised in rhs_inst.hip.
@@ -141,6 +165,7 @@ hipError_t launch_pack_left(const double* src, double* dst, const int cells[3], 
 // for Euler) and qbar [E][NV][NN].
 struct AdParams {
   KParams k;
+  double Ds[kMaxN1][kMaxN1], Dhat[kMaxN1][kMaxN1], inv_w[kMaxN1];  // as Operators
   const double* v;  // tangent direction or cotangent
   const double* x1;
   const double* x2;

@@ -350,8 +350,8 @@ __global__ void __launch_bounds__((Shape<DIM, N>::NN)) __attribute__((amdgpu_wav
       for (int c = 0; c < DIM; ++c) s_ja[(d * DIM + c) * PN + pa] = 0.5 * jm[d][c];
   }
   if (a < n * n) {
-    s_D[(a / n) * DS + a % n] = p.Ds[a / n][a % n];
-    s_Dh[(a / n) * DS + a % n] = p.Dhat[a / n][a % n];
+    s_D[(a / n) * DS + a % n] = p.basis[a];
+    s_Dh[(a / n) * DS + a % n] = p.basis[n * n + a];
   }
   __syncthreads();
 

@@ -114,9 +114,9 @@ __device__ __forceinline__ void node_metric(const KParams& p, int64_t e, const i
 // neighbours' (NV values, from grad_vars; overwritten); blo, bhi: the end is a
 // boundary face, whose value comes from the boundary condition; sg_*: sign(J) at
 // the line's end nodes (the face terms use the element's own normal).
-template <int DIM, int N, bool NODAL, bool BCS>
-__device__ __forceinline__ void line_gradient(const KParams& p, int64_t el, const int* eid, int dl,
-                                              int line, int first, int last,
+template <int DIM, int N, bool NODAL, bool BCS, class Ops>
+__device__ __forceinline__ void line_gradient(const KParams& p, const Ops& op, int64_t el,
+                                              const int* eid, int dl, int line, int first, int last,
                                               const double (&x)[N + 1][DIM + 1], double* q_lo,
                                               double* q_hi, bool blo, bool bhi, double sg_lo,
                                               double sg_hi, double (&acc)[N + 1][DIM + 1]) {
@@ -127,7 +127,7 @@ __device__ __forceinline__ void line_gradient(const KParams& p, int64_t el, cons
     for (int v = 0; v < ND; ++v) {
       double r = 0.0;
 #pragma unroll
-      for (int i = 0; i < n; ++i) r += p.Dhat[k][i] * x[i][v];
+      for (int i = 0; i < n; ++i) r += op.Dhat(k, i) * x[i][v];
       acc[k][v] = r;
     }
 #pragma unroll
@@ -242,8 +242,8 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) viscous_flux_ker
     double q_lo[NV], q_hi[NV];
     grad_vars<DIM>(p.gamma, t_lo, q_lo);
     grad_vars<DIM>(p.gamma, t_hi, q_hi);
-    line_gradient<DIM, N, NODAL, BCS>(p, el, eid, dl, line, first, last, x, q_lo, q_hi, blo, bhi,
-                                      sg_lo, sg_hi, acc);
+    line_gradient<DIM, N, NODAL, BCS>(p, Operators<N>(p), el, eid, dl, line, first, last, x, q_lo,
+                                      q_hi, blo, bhi, sg_lo, sg_hi, acc);
   }
   __syncthreads();  // every line has read its q
   if (dir < DIM) {
@@ -355,7 +355,7 @@ __global__ void __launch_bounds__((Shape<DIM, N>::NN)) gradient_node_kernel(cons
   grad_vars<DIM>(p.gamma, u, q);
 #pragma unroll
   for (int v = 0; v < NV; ++v) s_q[v * NN + a] = q[v];
-  if (a < n * n) s_Dh[a] = p.Dhat[a / n][a % n];
+  if (a < n * n) s_Dh[a] = p.basis[n * n + a];
   __syncthreads();
   double r[DIM][NV];
 #pragma unroll

@@ -146,6 +146,44 @@ __device__ __forceinline__ int xcd_block(int b, int nb) {
   return x * q + (x < r ? x : r) + i;
 }
 
+// Blending factor of an element from the modal energies: of all modes, without
+// the highest of each direction, and without the two highest
+// (indicator.hpp:337-417).
+__device__ __forceinline__ double blending_factor(const KParams& p, double total, double clip1,
+                                                  double clip2) {
+  const double ef1 = total != 0.0 ? (total - clip1) / total : 0.0;
+  const double ef2 = clip1 != 0.0 ? (clip1 - clip2) / clip1 : 0.0;
+  const double energy = dmax(ef1, ef2);
+  double a = 1.0 / (1.0 + exp(-p.sfac / p.threshold * (energy - p.threshold)));
+  if (a < p.alpha_min) a = 0.0;
+  if (a > 1.0 - p.alpha_min) a = 1.0;
+  return dmin(p.alpha_max, a);
+}
+
+// The SSPRK3 stage at a node, in place of its right-hand side r: c1 u_base + c2
+// u_k + c3 r (stage 3) or c1 u_k + c2 r, then the positivity floor.
+template <int DIM>
+__device__ __forceinline__ void stage_combine(const KParams& p, bool with_base, const double* uk,
+                                              const double* ub, double* r) {
+  constexpr int NV = DIM + 2;
+  if (with_base) {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) r[v] = p.c1 * ub[v] + p.c2 * uk[v] + p.c3 * r[v];
+  } else {
+#pragma unroll
+    for (int v = 0; v < NV; ++v) r[v] = p.c1 * uk[v] + p.c2 * r[v];
+  }
+  if (p.floor_value > 0.0) {
+    if (r[0] < p.floor_value) r[0] = p.floor_value;
+    double m2 = 0.0;
+#pragma unroll
+    for (int k = 0; k < DIM; ++k) m2 += r[k + 1] * r[k + 1];
+    const double kin = 0.5 * m2 / r[0];
+    if ((p.gamma - 1.0) * (r[NV - 1] - kin) < p.floor_value)
+      r[NV - 1] = p.floor_value / (p.gamma - 1.0) + kin;
+  }
+}
+
 // Hennemann-Gassner modal indicator for the EPW elements of the block,
 // indicator.hpp:337-417 (2D) / :454-574 (3D), including the 3D total-energy
 // sum that skips the modes (i = N, j < N, k < N) and gamma fixed at 1.4.
@@ -167,7 +205,7 @@ __device__ void block_alpha(const KParams& p, double* s_w, double* s_alpha, int 
   constexpr int n = S::n, NN = S::NN;
   constexpr int LN = NN / n;  // lines per direction and element
   double* A = s_w;
-  const double* V = p.Vinv;
+  const Operators<N> op(p);
   const int tid = threadIdx.x;
   // sweep along xi, lines of fixed (j, k)
   for (int t = tid; t < EPW * LN; t += BLOCK) {
@@ -179,7 +217,7 @@ __device__ void block_alpha(const KParams& p, double* s_w, double* s_alpha, int 
     for (int i = 0; i < n; ++i) {
       double r = 0.0;
 #pragma unroll
-      for (int ii = 0; ii < n; ++ii) r += V[i * n + ii] * x[ii];
+      for (int ii = 0; ii < n; ++ii) r += op.Vinv(i, ii) * x[ii];
       A[slot * S::SP + lds_pos<N>(row + i)] = r;
     }
   }
@@ -195,7 +233,7 @@ __device__ void block_alpha(const KParams& p, double* s_w, double* s_alpha, int 
     for (int j = 0; j < n; ++j) {
       double r = 0.0;
 #pragma unroll
-      for (int jj = 0; jj < n; ++jj) r += V[j * n + jj] * x[jj];
+      for (int jj = 0; jj < n; ++jj) r += op.Vinv(j, jj) * x[jj];
       A[slot * S::SP + lds_pos<N>(base + j * n)] = r;
     }
   }
@@ -212,7 +250,7 @@ __device__ void block_alpha(const KParams& p, double* s_w, double* s_alpha, int 
       for (int k = 0; k < n; ++k) {
         double r = 0.0;
 #pragma unroll
-        for (int kk = 0; kk < n; ++kk) r += V[k * n + kk] * x[kk];
+        for (int kk = 0; kk < n; ++kk) r += op.Vinv(k, kk) * x[kk];
         A[slot * S::SP + lds_pos<N>(base + k * n * n)] = r;
       }
     }
@@ -246,13 +284,7 @@ __device__ void block_alpha(const KParams& p, double* s_w, double* s_alpha, int 
       for (int k = 0; k < n - 1; ++k)
         for (int i = 0; i < n; ++i) total += M(k, n - 1, i) * M(k, n - 1, i);
     }
-    const double ef1 = total != 0.0 ? (total - clip1) / total : 0.0;
-    const double ef2 = clip1 != 0.0 ? (clip1 - clip2) / clip1 : 0.0;
-    const double energy = dmax(ef1, ef2);
-    double a = 1.0 / (1.0 + exp(-p.sfac / p.threshold * (energy - p.threshold)));
-    if (a < p.alpha_min) a = 0.0;
-    if (a > 1.0 - p.alpha_min) a = 1.0;
-    s_alpha[tid] = dmin(p.alpha_max, a);
+    s_alpha[tid] = blending_factor(p, total, clip1, clip2);
   }
   __syncthreads();
 }
