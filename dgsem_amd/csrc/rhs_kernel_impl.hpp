@@ -421,6 +421,7 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES))
 }  // namespace dgsem
 
 #include "node_kernel_impl.hpp"
+#include "pair_kernel_impl.hpp"
 
 namespace dgsem {
 namespace detail {
@@ -430,6 +431,10 @@ hipError_t launch_one(const KParams& p, hipStream_t stream) {
   static_assert(SF != kFluxAny || (DIM == 2 && N <= 5), "run-time fluxes: 2D line kernels");
   if constexpr (SF != kFluxAny && use_node_kernel<DIM, N, SC, BCS>())
     return launch_node_kernel<DIM, N, NODAL, SF>(p, stream);
+  if constexpr (DIM == 2 && !use_node_kernel<DIM, N, SC, BCS>()) {
+    if (pair_kernel_for<N, SF, FF>(p.E, p.visc != nullptr))
+      return launch_pair_kernel<N, SC, NODAL, SF, FF, BCS>(p, stream);
+  }
   constexpr int EPW = elems_per_block<DIM, N>();
   constexpr int BLOCK = EPW * Shape<DIM, N>::LINES;
   const int64_t nb = (p.E + EPW - 1) / EPW;
