@@ -409,8 +409,8 @@ int dgsem_create(const dgsem_config* cfg, void* stream, dgsem_handle** out) {
     *out = h;
     return rc;
   }
-  // periodic nodal box meshes: the metric terms' table for the line kernels
-  if (h->cfg.geometry == DGSEM_GEOMETRY_NODAL && !has_boundaries(h->cfg)) {
+  // nodal box meshes: the metric terms' table
+  if (h->cfg.geometry == DGSEM_GEOMETRY_NODAL) {
     std::vector<double> tab;
     if (dgsem::box_metric_table(h->geo, tab, h->ja_box_off) && (rc = upload(h, &h->d_ja_box, tab))) {
       release(h);

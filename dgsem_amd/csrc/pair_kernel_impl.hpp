@@ -19,8 +19,8 @@
 // The sums run in the line kernel's order on the same operations (surface terms,
 // pairs by the other node, subcell faces, viscous terms; then direction 0 +
 // direction 1), so both kernels give the same bits and the choice between them
-// (pair_kernel_for) cannot be seen in the results.  Bounded by latency: of the 7 us
-// a launch takes at 16 x 16, N = 3 (12 in the line kernel), 1.7 are an empty
+// (pair_kernel_for) cannot be seen in the results.  Bounded by latency: of the 6.4
+// us a launch takes at 16 x 16, N = 3 (11.7 in the line kernel), 1.7 are an empty
 // launch's and 0.7 a copy's; then come one flux, the indicator and the sums, each
 // behind a barrier.
 #pragma once
@@ -119,8 +119,10 @@ __device__ __forceinline__ void wave_alpha(const KParams& p, double w, const dou
   if (lane < W::EPW) s_alpha[lane] = blending_factor(p, total, clip1, clip2);
 }
 
-// BOX: NODAL metric terms from the box-mesh table (periodic meshes).
-template <int N, bool SC, bool NODAL, int SF, int FF, bool BCS, bool BOX>
+// The metric terms come from the full arrays on box meshes too: at these sizes
+// the table of the larger grids (box_table_for) saves no time on memory and its
+// addresses cost 2%.
+template <int N, bool SC, bool NODAL, int SF, int FF, bool BCS>
 __global__ void __launch_bounds__(PairShape<N>::BLOCK)
     __attribute__((amdgpu_waves_per_eu(pair_waves_per_simd<N, SF, FF>())))
     rhs_pair_kernel(const KParams p) {
@@ -162,15 +164,7 @@ __global__ void __launch_bounds__(PairShape<N>::BLOCK)
 #pragma unroll
     for (int v = 0; v < NV; ++v) u[v] = src[v * NN];
     double ja[4];
-    if constexpr (BOX) {
-      int eid[3];
-      element_indices<2>(p, (int)e, eid);
-#pragma unroll
-      for (int c = 0; c < 2; ++c) {
-        ja[c] = box_row<2, N>(p, eid, c, 0, nj)[ni];
-        ja[2 + c] = box_row<2, N>(p, eid, c, 1, ni)[nj];
-      }
-    } else if constexpr (NODAL) {
+    if constexpr (NODAL) {
 #pragma unroll
       for (int k = 0; k < 4; ++k) ja[k] = 0.5 * p.Ja[(e * 4 + k) * NN + node];
     }
@@ -208,22 +202,10 @@ __global__ void __launch_bounds__(PairShape<N>::BLOCK)
     const double* src = p.u + (boundary ? fe : nb) * (NV * NN) + (fside ? first : last);
 #pragma unroll
     for (int v = 0; v < NV; ++v) far[v] = src[v * NN];
-    if constexpr (BOX) {
-      if (fside) {  // the upper neighbour's indices differ in direction fdir only
+    const double sg = p.invJ[NODAL ? ue * NN + at : ue] >= 0.0 ? 1.0 : -1.0;
 #pragma unroll
-        for (int r = 0; r < 2; ++r) {
-          const int up = fid[r] + 1 != p.cells[r] ? fid[r] + 1 : 0;
-          fid[r] = r == fdir ? up : fid[r];
-        }
-      }
-#pragma unroll
-      for (int c = 0; c < 2; ++c) nrm_f[c] = 2.0 * box_row<2, N>(p, fid, c, fdir, fline)[0];
-    } else {
-      const double sg = p.invJ[NODAL ? ue * NN + at : ue] >= 0.0 ? 1.0 : -1.0;
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-        nrm_f[c] = sg * p.Ja[NODAL ? ((ue * 2 + fdir) * 2 + c) * NN + at : (ue * 2 + fdir) * 2 + c];
-    }
+    for (int c = 0; c < 2; ++c)
+      nrm_f[c] = sg * p.Ja[NODAL ? ((ue * 2 + fdir) * 2 + c) * NN + at : (ue * 2 + fdir) * 2 + c];
   }
   if (wave > 0 && wave <= W::PAIR_WAVES)
     for (int t = tid - 64; t < 3 * NN + n; t += 64 * W::PAIR_WAVES) s_op[t] = p.basis[t];
@@ -248,13 +230,10 @@ __global__ void __launch_bounds__(PairShape<N>::BLOCK)
         if (own_hi) hi_end = carried(2 * dir + 1);
       }
       const LineNodes<2, N> ln(dir, line);
-      double sg_lo = 1.0, sg_hi = 1.0;
-      if constexpr (!BOX) {
-        const int64_t ue = own_hi ? e : hi;
-        const int at = ln.base + (own_hi ? N * ln.stride : 0);
-        sg_lo = p.invJ[NODAL ? e * NN + ln.base : e] >= 0.0 ? 1.0 : -1.0;
-        sg_hi = p.invJ[NODAL ? ue * NN + at : ue] >= 0.0 ? 1.0 : -1.0;
-      }
+      const int64_t ue = own_hi ? e : hi;
+      const int at = ln.base + (own_hi ? N * ln.stride : 0);
+      const double sg_lo = p.invJ[NODAL ? e * NN + ln.base : e] >= 0.0 ? 1.0 : -1.0;
+      const double sg_hi = p.invJ[NODAL ? ue * NN + at : ue] >= 0.0 ? 1.0 : -1.0;
       const double* h = p.visc + (e * 2 + dir) * (NV * NN) + line * n;
       const double* hu = own_hi ? h + N : p.visc + (hi * 2 + dir) * (NV * NN) + line * n;
       double dh[n];
@@ -458,14 +437,7 @@ hipError_t launch_pair_kernel(const KParams& p, hipStream_t stream) {
   using W = PairShape<N>;
   const int64_t nb = (p.E + W::EPW - 1) / W::EPW;
   if (nb <= 0) return hipSuccess;
-  if constexpr (NODAL && !BCS) {
-    if (p.ja_box) {
-      hipLaunchKernelGGL((rhs_pair_kernel<N, SC, true, SF, FF, false, true>), dim3((unsigned)nb),
-                         dim3(W::BLOCK), 0, stream, p);
-      return hipGetLastError();
-    }
-  }
-  hipLaunchKernelGGL((rhs_pair_kernel<N, SC, NODAL, SF, FF, BCS, false>), dim3((unsigned)nb), dim3(W::BLOCK),
+  hipLaunchKernelGGL((rhs_pair_kernel<N, SC, NODAL, SF, FF, BCS>), dim3((unsigned)nb), dim3(W::BLOCK),
                      0, stream, p);
   return hipGetLastError();
 }

@@ -439,8 +439,8 @@ hipError_t launch_parabolic_t(bool sc, const KParams& p, hipStream_t s) {
       return hipGetLastError();
     }
   }
-  if constexpr (NODAL && !BCS) {
-    if (p.ja_box) {
+  if constexpr (NODAL) {
+    if (p.ja_box && box_table_for<DIM, N>(p.E)) {
       hipLaunchKernelGGL((viscous_flux_kernel<DIM, N, EPW, NODAL, BCS, true>), dim3((unsigned)nb),
                          dim3(BLOCK), 0, s, p);
       return hipGetLastError();

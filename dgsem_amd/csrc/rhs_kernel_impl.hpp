@@ -76,6 +76,18 @@ __device__ __forceinline__ const double* box_row(const KParams& p, const int* ei
   return p.ja_box + p.ja_box_off[c] + (uint64_t)(pair * DIM + r) * NN + line * n;
 }
 
+// Whether a box mesh's nodal metric terms are read from the table: it takes the
+// metrics' traffic off the memory, at the price of the table's addresses, which
+// a 2D grid that leaves the kernels waiting on latency does not earn back (line
+// kernel with boundaries, full arrays -> table, us a launch: N = 5 64 x 64
+// 12.3 -> 13.3, 96 x 96 21.9 -> 21.4, 128 x 128 35.8 -> 34.5; N = 3 96 x 96
+// 11.0 -> 11.7, 128 x 128 15.4 -> 14.5; periodic, table -> full arrays: N = 3
+// 96 x 96 8.6 -> 8.0).
+template <int DIM, int N>
+constexpr bool box_table_for(int64_t E) {
+  return DIM == 3 || E * Shape<DIM, N>::LINES >= 100000;
+}
+
 // Elements per workgroup: keeps EPW * LINES near 192 threads.
 template <int DIM, int N>
 constexpr int elems_per_block() {
@@ -395,7 +407,7 @@ template <int DIM, int N, int EPW, bool SC, bool NODAL, int SF, int FF, bool BCS
 __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES))
     __attribute__((amdgpu_waves_per_eu(min_waves_per_simd<DIM, N, NODAL>())))
     rhs_kernel(const KParams p) {
-  static_assert(!BOX || (NODAL && !BCS), "box-mesh tables serve periodic nodal meshes");
+  static_assert(!BOX || NODAL, "box-mesh tables hold nodal metric terms");
   using S = Shape<DIM, N>;
   constexpr int n = S::n, NV = S::NV, NN = S::NN, FN = S::FN, L = S::LINES, NP = S::NP;
   constexpr int BLOCK = EPW * L;
@@ -440,9 +452,8 @@ hipError_t launch_one(const KParams& p, hipStream_t stream) {
   const int64_t nb = (p.E + EPW - 1) / EPW;
   if (nb <= 0) return hipSuccess;
   if (nb > INT32_MAX) return hipErrorInvalidValue;
-  // nodal metric terms of a periodic box mesh come from the box table
-  if constexpr (NODAL && !BCS) {
-    if (p.ja_box) {
+  if constexpr (NODAL) {
+    if (p.ja_box && box_table_for<DIM, N>(p.E)) {
       hipLaunchKernelGGL((rhs_kernel<DIM, N, EPW, SC, NODAL, SF, FF, BCS, true>), dim3((unsigned)nb),
                          dim3(BLOCK), 0, stream, p);
       return hipGetLastError();
