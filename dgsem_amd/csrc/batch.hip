@@ -16,6 +16,8 @@
 #include "handle.hpp"
 #include "kernels.hpp"
 
+constexpr int kGridPerTile = INT32_MAX;  // capped by the number of tiles
+
 struct dgsem_batch {
   std::vector<dgsem_handle*> cases;
   std::vector<int64_t> offset, count;  // doubles of each case in a state arena
@@ -28,10 +30,15 @@ struct dgsem_batch {
   std::vector<double> dt;
   bool dt_set = false;
   // tuning: workgroup size, elements per tile for each N, persistent
-  // workgroups (0 = as many as fit the device at once)
-  int block = 256;
+  // workgroups (0 = as many as fit the device at once).  A new batch takes one
+  // workgroup of 128 threads per tile: LDS holds five of them on a CU (ten waves;
+  // two of 256 threads, eight), and the dispatcher places each as a CU comes
+  // free, where a persistent grid's round of unequal tiles ends with idle CUs.
+  // 64 cases of N = 2..5, two SSPRK3 steps on one MI355X: 256 threads persistent
+  // 404 us, one per tile 403; 128 threads persistent 442, one per tile 362.
+  int block = 128;
   int tile[8] = {0};
-  int grid = 0;
+  int grid = kGridPerTile;
   // derived launch state
   dgsem::BatchTile* d_tiles = nullptr;
   int ntiles = 0;
@@ -382,20 +389,22 @@ int dgsem_batch_autotune(dgsem_batch* b, const double* u, double* scratch, int r
     return er == hipSuccess ? DGSEM_OK : bhip(b, er, "timing");
   };
   int rc = DGSEM_OK;
-  int best_block = b->block, best_tile[8];
+  int best_block = b->block, best_grid = 0, best_tile[8];
   std::memcpy(best_tile, b->tile, sizeof(best_tile));
   float best = 1e30f;
-  for (int blk : dgsem::kBatchBlocks) {
-    int zero[8] = {0};
-    if ((rc = dgsem_batch_set_tuning(b, blk, zero, 0))) break;
-    float ms = 0;
-    if ((rc = measure(&ms))) break;
-    if (ms < best) {
-      best = ms;
-      best_block = blk;
-      std::memcpy(best_tile, zero, sizeof(best_tile));
+  for (int blk : dgsem::kBatchBlocks)
+    for (int grid : {0, kGridPerTile}) {
+      int zero[8] = {0};
+      if (rc != DGSEM_OK || (rc = dgsem_batch_set_tuning(b, blk, zero, grid))) break;
+      float ms = 0;
+      if ((rc = measure(&ms))) break;
+      if (ms < best) {
+        best = ms;
+        best_block = blk;
+        best_grid = grid;
+        std::memcpy(best_tile, zero, sizeof(best_tile));
+      }
     }
-  }
   std::vector<int> degrees;
   for (dgsem_handle* h : b->cases)
     if (std::find(degrees.begin(), degrees.end(), h->cfg.polydeg) == degrees.end())
@@ -409,7 +418,7 @@ int dgsem_batch_autotune(dgsem_batch* b, const double* u, double* scratch, int r
       int trial[8];
       std::memcpy(trial, best_tile, sizeof(trial));
       trial[N] = t;
-      if ((rc = dgsem_batch_set_tuning(b, best_block, trial, 0))) break;
+      if ((rc = dgsem_batch_set_tuning(b, best_block, trial, best_grid))) break;
       float ms = 0;
       if ((rc = measure(&ms))) break;
       if (ms < best) {
@@ -418,7 +427,6 @@ int dgsem_batch_autotune(dgsem_batch* b, const double* u, double* scratch, int r
       }
     }
   }
-  int best_grid = 0;
   if (rc == DGSEM_OK) {
     if ((rc = dgsem_batch_set_tuning(b, best_block, best_tile, 0)) == DGSEM_OK) {
       const int full = b->grid_eff;

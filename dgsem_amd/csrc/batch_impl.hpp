@@ -4,7 +4,8 @@
 // The host cuts every case into tiles of at most EPW(N) consecutive
 // elements (EPW(N) = BLOCK / LINES(N) element slots fit one workgroup) and
 // sorts the tiles by degree, highest first, and by estimated cost within a
-// degree.  Each workgroup walks the tile list with a grid-size stride; a
+// degree.  Each workgroup walks the tile list with a grid-size stride (by
+// default the grid has a workgroup per tile, see batch.hip); a
 // tile names its case, whose KParams (state, geometry, basis and stage
 // coefficients) sit in a device array, and the degree's loop it falls in
 // selects the instantiation of the element body.  The element body is the

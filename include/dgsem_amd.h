@@ -334,7 +334,8 @@ int dgsem_batch_rhs(dgsem_batch* b, const double* u, double* du);
 int dgsem_batch_ssprk3_steps(dgsem_batch* b, double* u, int nsteps, double* tmp1, double* tmp2);
 /* Tuning: workgroup size (128 or 256), elements per tile for each degree
  * (tile_elems[N], N = 0..7; 0 = as many as one workgroup holds) and the
- * number of persistent workgroups (0 = all that fit the device at once). */
+ * number of persistent workgroups (0 = all that fit the device at once).  A
+ * new batch takes 128 threads and one workgroup per tile. */
 int dgsem_batch_get_tuning(const dgsem_batch* b, int* block, int* tile_elems, int* grid);
 int dgsem_batch_set_tuning(dgsem_batch* b, int block, const int* tile_elems, int grid);
 /* Autotuner: times the batch RHS of u (written to `scratch`, an arena) over
