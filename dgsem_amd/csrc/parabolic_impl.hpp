@@ -422,7 +422,7 @@ __global__ void __launch_bounds__((Shape<DIM, N>::NN)) gradient_node_kernel(cons
 
 template <int DIM, int N>
 constexpr int parabolic_elems_per_block() {
-  constexpr int e = 192 / Shape<DIM, N>::LINES;
+  constexpr int e = (DIM == 2 ? 64 : 192) / Shape<DIM, N>::LINES;  // as elems_per_block
   return e < 1 ? 1 : e;
 }
 

@@ -88,11 +88,16 @@ constexpr bool box_table_for(int64_t E) {
   return DIM == 3 || E * Shape<DIM, N>::LINES >= 100000;
 }
 
-// Elements per workgroup: keeps EPW * LINES near 192 threads.
+// Elements per workgroup: keeps EPW * LINES near 192 threads in 3D and within one
+// wave in 2D.  A 2D element has few lines, so blocks of one wave fill the CUs
+// evenly (LDS holds about ten waves either way) and wait for no other wave.
+// Launches of 192-thread blocks -> one wave, us: Kelvin-Helmholtz N = 3 128 x 128
+// 12.8 -> 11.7, N = 5 112 x 112 27.9 -> 24.3, N = 7 80 x 80 37.4 -> 27.4; Riemann
+// problem N = 5 112 x 112 29.4 -> 24.3; 5% on the average of 48 x 48 to 160 x 160.
 template <int DIM, int N>
 constexpr int elems_per_block() {
   constexpr int L = Shape<DIM, N>::LINES;
-  constexpr int e = 192 / L;
+  constexpr int e = (DIM == 2 ? 64 : 192) / L;
   return e < 1 ? 1 : e;
 }
 
