@@ -164,7 +164,7 @@ def cpu_baseline(N: int, cells: int, steps: int, warmup: int) -> dict:
 def batch_measure(ncases: int = 256, steps: int = 100, seed: int = 2024, sequential: bool = True) -> dict:
     """Ensemble of 2D Kelvin-Helmholtz cases (grids from {8,16,32,64}^2, N from
     {2,3,4,5}): `steps` SSPRK3 steps of the autotuned batch (graph replay of
-    one persistent launch per stage) against the same steps run case after
+    one launch per stage) against the same steps run case after
     case with the single-case handles; per-case results compared bitwise.
     sequential=False times the batch alone (for profiling it).
 

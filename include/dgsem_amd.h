@@ -305,7 +305,7 @@ int dgsem_write_vtu(dgsem_handle* h, const double* u, const char* path);
  * one StructuredSolver per process, one case after another.  A batch
  * advances many independent 2D Euler cases (different element grids and
  * polynomial degrees; one volume integral, flux pair and geometry mode for
- * all) with one persistent kernel launch per SSPRK3 stage, the three stages
+ * all) with one kernel launch per SSPRK3 stage, the three stages
  * of a step recorded once into a HIP graph.  Each case gives bit-identical
  * results to its own single-case handle (dgsem_ssprk3_steps).
  *
