@@ -916,16 +916,17 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES)) vjp_viscous_kern
   }
 }
 
-// Whether the adjoint kernel forms the subcell cotangents of all directions
-// at once: in 3D up to N = 3, where the per-direction arrays keep the LDS of
-// a block within 80 KiB, so the two blocks per CU its registers allow still
-// fit.  (With HLLC subcells and every element troubled, 3D N = 3 at 32^3,
-// the adjoint took 5.7 ms with one direction at a time.)
-template <int DIM, int N, int EPW, bool SC>
+// Whether the adjoint kernel forms the subcell cotangents of all directions at
+// once: in 3D up to N = 3, where a line's n NV cotangents fit the registers its
+// other sums have left.  They wait there for their direction's turn to be added, so
+// the LDS (40 KB a block at N = 3) holds nothing for them.  32^3, N = 3, one
+// direction at a time -> all at once, us an adjoint right-hand side with every
+// element troubled: LLF 382 -> 282, HLLC 600 -> 430, viscous 571 -> 477 and 1175 ->
+// 630; with none troubled 195 -> 195, 286 -> 287, 394 -> 396 and 655 -> 492 (the
+// serial pass took the viscous HLLC kernel past 256 registers).  16^3: 13-40% less.
+template <int DIM, int N>
 constexpr bool par_subcell_adjoint() {
-  using S = Shape<DIM, N>;
-  constexpr int lds = 8 * EPW * S::PN * (DIM + 2 + 2 * S::NV + S::NV - 1 + DIM * S::NV);
-  return SC && DIM == 3 && N <= 3 && lds <= 80 * 1024;
+  return DIM == 3 && N <= 3;
 }
 
 template <int DIM, int N, int EPW, bool NODAL, bool NS, bool SC, int SF, int FF>
@@ -948,11 +949,9 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES))
   __shared__ double s_qv[NS ? EPW * SD : 1];
   double* const s_qb = s_p;
   double* const s_ub = SC ? s_ub_own : s_r;
-  // PAR_FV (shock capturing, where the LDS allows): the troubled elements'
-  // subcell cotangents are formed by all directions' lines at once, into
-  // one array per direction, instead of one direction at a time.
-  constexpr bool PAR_FV = par_subcell_adjoint<DIM, N, EPW, SC>();
-  __shared__ double s_fv[PAR_FV ? DIM * EPW * SU : 1];
+  // PAR_FV: the troubled elements' subcell cotangents are formed by all
+  // directions' lines at once instead of one direction at a time.
+  constexpr bool PAR_FV = SC && par_subcell_adjoint<DIM, N>();
   const int tid = threadIdx.x;
   const int64_t e0 = (int64_t)xcd_block(blockIdx.x, gridDim.x) * EPW;
   const int nvalid = (int)((p.E - e0) < EPW ? (p.E - e0) : EPW);
@@ -1005,6 +1004,14 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES))
   double qv[NS ? n : 1][ND];
   double coef = 1.0, alpha = 0.0;
   const bool troubled = l.valid && frozen_blend<SC>(p, l.e, coef, alpha);
+  bool any = false;  // an element of the block is troubled (uniform)
+  if constexpr (PAR_FV) {
+#pragma unroll
+    for (int sl = 0; sl < EPW; ++sl) {
+      double cf, al;
+      any = frozen_blend<SC>(p, e0 + (sl < nvalid ? sl : nvalid - 1), cf, al) || any;
+    }
+  }
   if (l.valid) {
     const double* rr = s_r + l.slot * SU;
     // faces: this element's share of each face flux's adjoint
@@ -1242,40 +1249,50 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES))
     }
     __syncthreads();
   }
-  // PAR_FV: the same subcell terms, all directions at once now that the
-  // line's other sums are in LDS.  Each direction has its own array, where
-  // the line owns its nodes: node fi - 1 gets its second term here, node fi
-  // its first.
+  // PAR_FV: the same subcell terms, formed by all directions' lines at once now
+  // that the line's other sums are in LDS (and their registers free), then added
+  // one direction at a time.
   if constexpr (PAR_FV) {
-    if (troubled) {
-      const double* rr = s_r + l.slot * SU;
-      double* fvp = s_fv + (l.dir * EPW + l.slot) * SU;
-#pragma unroll 1
-      for (int fi = 1; fi < n; ++fi) {
-        double ul[NV], ur[NV], nrm[DIM], g[NV], ubl[NV], ubr[NV];
-        load_state<DIM, NN>(p.u, l.e, l.dof(fi - 1), ul);
-        load_state<DIM, NN>(p.u, l.e, l.dof(fi), ur);
-        subcell_normal<DIM, N, NODAL>(p, l.e, l.dir, l.line, fi - 1, nrm);
-        const double wl = alpha * op.inv_w(fi - 1), wr = alpha * op.inv_w(fi);
-        for (int v = 0; v < NV; ++v) {
-          g[v] = wl * rr[v * PN + l.pos(fi - 1)] - wr * rr[v * PN + l.pos(fi)];
-          ubl[v] = ubr[v] = 0.0;
-        }
-        if constexpr (FF == kFluxHLLC) {
-          hllc_vjp<DIM>(p.gamma, ul, ur, nrm, g, true, true, ubl, ubr);
-        } else {
-          const NodePrims<DIM> ql = node_prims<DIM>(p.gamma, ul), qr = node_prims<DIM>(p.gamma, ur);
-          llf_vjp_side<DIM>(p.gamma, ul, ql, ur, qr, nrm, g, true, ubl);
-          llf_vjp_side<DIM>(p.gamma, ul, ql, ur, qr, nrm, g, false, ubr);
-        }
-        for (int v = 0; v < NV; ++v) {
-          double* lo = fvp + v * PN + l.pos(fi - 1);
-          *lo = fi == 1 ? ubl[v] : *lo + ubl[v];
-          fvp[v * PN + l.pos(fi)] = ubr[v];
+    if (any) {
+      double fv[n][NV];
+#pragma unroll
+      for (int k = 0; k < n; ++k)
+#pragma unroll
+        for (int v = 0; v < NV; ++v) fv[k][v] = 0.0;
+      if (troubled) {
+        const double* rr = s_r + l.slot * SU;
+#pragma unroll
+        for (int fi = 1; fi < n; ++fi) {
+          double ul[NV], ur[NV], nrm[DIM], g[NV];
+          load_state<DIM, NN>(p.u, l.e, l.dof(fi - 1), ul);
+          load_state<DIM, NN>(p.u, l.e, l.dof(fi), ur);
+          subcell_normal<DIM, N, NODAL>(p, l.e, l.dir, l.line, fi - 1, nrm);
+          const double wl = alpha * op.inv_w(fi - 1), wr = alpha * op.inv_w(fi);
+#pragma unroll
+          for (int v = 0; v < NV; ++v)
+            g[v] = wl * rr[v * PN + l.pos(fi - 1)] - wr * rr[v * PN + l.pos(fi)];
+          if constexpr (FF == kFluxHLLC) {
+            hllc_vjp<DIM>(p.gamma, ul, ur, nrm, g, true, true, fv[fi - 1], fv[fi]);
+          } else {
+            const NodePrims<DIM> ql = node_prims<DIM>(p.gamma, ul), qr = node_prims<DIM>(p.gamma, ur);
+            llf_vjp_side<DIM>(p.gamma, ul, ql, ur, qr, nrm, g, true, fv[fi - 1]);
+            llf_vjp_side<DIM>(p.gamma, ul, ql, ur, qr, nrm, g, false, fv[fi]);
+          }
+          pin_values<NV>(fv[fi - 1]);
+          pin_values<NV>(fv[fi]);
         }
       }
+#pragma unroll
+      for (int d = 0; d < DIM; ++d) {
+        if (troubled && l.dir == d) {
+#pragma unroll
+          for (int k = 0; k < n; ++k)
+#pragma unroll
+            for (int v = 0; v < NV; ++v) s_ub[l.slot * SU + v * PN + l.pos(k)] += fv[k][v];
+        }
+        __syncthreads();
+      }
     }
-    __syncthreads();
   }
   for (int i = tid; i < NODES; i += BLOCK) {
     const int sl = i / NN, node = i - sl * NN, pn = lds_pos<N>(node);
@@ -1293,13 +1310,6 @@ __global__ void __launch_bounds__((EPW * Shape<DIM, N>::LINES))
     qbar.kin = 0.0;  // the pair flux does not take it
 #pragma unroll
     for (int v = 0; v < NV; ++v) ub[v] = s_ub[sl * SU + v * PN + pn];
-    if constexpr (PAR_FV) {
-      double cf, al;
-      if (frozen_blend<SC>(p, e, cf, al)) {
-        for (int d = 0; d < DIM; ++d)
-          for (int v = 0; v < NV; ++v) ub[v] += s_fv[(d * EPW + sl) * SU + v * PN + pn];
-      }
-    }
     prims_vjp<DIM>(p.gamma, q, qbar, 0.0, ub);
     if constexpr (NS) {
       double x[NV];
