@@ -287,6 +287,16 @@ __device__ __forceinline__ void flux_hllc_exact(double g, const double* ul, cons
   for (int i = 0; i < NV; ++i) f[i] *= nrm;
 }
 
+// The face fluxes of an element, one per line end, and the rounds in which its NN
+// threads form them: thread a takes line end a + k NN in round k.  From N = 5 in 3D
+// and N = 3 in 2D on there is a thread for each; a kernel built for lower degrees
+// (DGSEM_NODE_KERNEL_MIN_N) takes further rounds.
+template <int DIM, int N>
+struct NodeFaces {
+  static constexpr int NN = Shape<DIM, N>::NN, COUNT = 2 * DIM * Shape<DIM, N>::FN;
+  static constexpr int ROUNDS = (COUNT + NN - 1) / NN;
+};
+
 template <int DIM, int N, bool NODAL, int SF>
 __global__ void __launch_bounds__((Shape<DIM, N>::NN)) __attribute__((amdgpu_waves_per_eu(4)))
     rhs_node_kernel(const KParams p) {
@@ -295,11 +305,11 @@ __global__ void __launch_bounds__((Shape<DIM, N>::NN)) __attribute__((amdgpu_wav
   constexpr int DS = n + 1;        // padded row of the D_split table
   constexpr int QB = DIM + 1;      // plane of beta; kin follows
   constexpr int FN = Shape<DIM, N>::FN;
-  constexpr int FACE = 2 * DIM * FN;  // face fluxes of the element, one per line end
+  using Faces = NodeFaces<DIM, N>;
   // LDS planes: rho, v[DIM], beta, kin, then (NODAL) Ja^d_c / 2.  Once the term
   // loops are done with them they take the face fluxes (FPL planes) and the
   // viscous fluxes (VPL planes: the mass component is zero).
-  constexpr int QPL = DIM + 3, FPL = (FACE * NV + PN - 1) / PN, VPL = DIM * (NV - 1);
+  constexpr int QPL = DIM + 3, FPL = (Faces::COUNT * NV + PN - 1) / PN, VPL = DIM * (NV - 1);
   constexpr int JPL = NODAL ? DIM * DIM : 0;
   constexpr int PLANES = QPL + JPL > FPL + VPL ? QPL + JPL : FPL + VPL;
   __shared__ double s_q[PLANES * PN];
@@ -426,18 +436,20 @@ __global__ void __launch_bounds__((Shape<DIM, N>::NN)) __attribute__((amdgpu_wav
   }
 
   // 4. numerical fluxes on the element's faces, one thread for each line end:
-  // thread (dir, side, line) of the first FACE threads, so that a wave takes
-  // one side of one direction (3D) and every lane works.  Formed by the face
+  // item (dir, side, line) to a thread (NodeFaces), so that a wave takes one side
+  // of one direction (3D) and every lane works.  Formed by the face
   // nodes' own threads they ran once per direction in every wave, a quarter of
   // its lanes active.  The lower face takes the lower neighbour's node with
   // index N, the upper face the upper neighbour's node with index 0 and its
   // metric row and 1/J, whose sign and row make the interface normal.
   {
-    const bool has_face = a < FACE;
-    const int fd = a / (2 * FN), rem = a - fd * (2 * FN), line = rem % FN;
-    const bool lower = rem < FN;
-    double f[NV];
-    if (has_face) {
+    double f[Faces::ROUNDS][NV];
+#pragma unroll
+    for (int k = 0; k < Faces::ROUNDS; ++k) {
+      const int t = a + k * NN;
+      if (t >= Faces::COUNT) break;
+      const int fd = t / (2 * FN), rem = t - fd * (2 * FN), line = rem % FN;
+      const bool lower = rem < FN;
       const LineNodes<DIM, N> ln(fd, line);
       const int first = ln.base, last = ln.base + N * ln.stride;
       int64_t lo, hi;
@@ -466,15 +478,19 @@ __global__ void __launch_bounds__((Shape<DIM, N>::NN)) __attribute__((amdgpu_wav
         ur[v] = lower ? so[v] : sn[v];
       }
       if constexpr (SF == kFluxLLF) {
-        flux_llf_exact<DIM>(p.gamma, ul, ur, nrm, f);
+        flux_llf_exact<DIM>(p.gamma, ul, ur, nrm, f[k]);
       } else {
-        flux_hllc_exact<DIM>(p.gamma, ul, ur, nrm, f);
+        flux_hllc_exact<DIM>(p.gamma, ul, ur, nrm, f[k]);
       }
     }
     __syncthreads();  // the term loops are done with the primitives
-    if (has_face) {
 #pragma unroll
-      for (int v = 0; v < NV; ++v) s_face[((fd * 2 + (lower ? 0 : 1)) * NV + v) * FN + line] = f[v];
+    for (int k = 0; k < Faces::ROUNDS; ++k) {
+      const int t = a + k * NN;
+      if (t >= Faces::COUNT) break;
+      const int face = t / FN, line = t % FN;  // face = 2 dir + upper
+#pragma unroll
+      for (int v = 0; v < NV; ++v) s_face[(face * NV + v) * FN + line] = f[k][v];
     }
   }
 
