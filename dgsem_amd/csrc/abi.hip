@@ -196,6 +196,7 @@ void fill_params(dgsem_handle* h) {
     for (int v = 0; v < 5; ++v) p.bc_state[f][v] = c.face_state[f][v];
     p.bc_values[f] = nullptr;
   }
+  p.cus = h->cus;
 }
 
 // Per-face boundary kinds: a face left at 0 takes boundary[its direction].
@@ -377,7 +378,8 @@ int dgsem_create(const dgsem_config* cfg, void* stream, dgsem_handle** out) {
     return rc;
   }
   h->stream = (hipStream_t)stream;
-  if (hipGetDevice(&h->device) != hipSuccess) {
+  if (hipGetDevice(&h->device) != hipSuccess ||
+      hipDeviceGetAttribute(&h->cus, hipDeviceAttributeMultiprocessorCount, h->device) != hipSuccess) {
     *out = h;
     return fail(h, DGSEM_E_HIP, "no HIP device");
   }

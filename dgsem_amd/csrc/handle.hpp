@@ -16,6 +16,7 @@ struct dgsem_handle {
   dgsem::Geometry geo;
   hipStream_t stream = nullptr;
   int device = 0;
+  int cus = 0;  // compute units of the device
   int nvars = 0, nn = 0;
   int64_t E = 0;
   // device buffers

@@ -99,6 +99,7 @@ struct KParams {
   int bc[6];
   double bc_state[6][5];
   const double* bc_values[6];
+  int cus;               // compute units of the device, for the launchers' choice of kernel
 };
 
 // The basis operators of N + 1 = n nodes at KParams::basis: D_split, D_hat and

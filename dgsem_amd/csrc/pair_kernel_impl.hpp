@@ -49,12 +49,12 @@ constexpr int pair_waves_per_simd() {
   return SF == kFluxLLF && FF == kFluxLLF && N != 7 ? 6 : 5;
 }
 
-// The pair kernel serves grids whose blocks all fit the chip at once (N = 7: twice
-// over): beyond that its waves queue, while the line kernel, with fewer
+// The pair kernel serves grids whose blocks all fit the device's CUs at once (N = 7:
+// twice over): beyond that its waves queue, while the line kernel, with fewer
 // instructions per flux, still fits.  The HLLC kinds fill five waves per SIMD
 // badly, and with viscous terms the viscous kernel takes a share of the gain:
-// 16 waves per CU for both.  Times per launch at the sides of the line, line
-// kernel -> this one (us; Kelvin-Helmholtz with the indicator, LLF):
+// 16 waves per CU for both.  Times per launch at the sides of the line on 256 CUs,
+// line kernel -> this one (us; Kelvin-Helmholtz with the indicator, LLF):
 //   N = 1 (24576 elements)  128 x 128: 7.1 -> 6.6    160 x 160:  8.5 ->  9.0
 //   N = 2 (7168)              64 x 64: 8.4 -> 7.8      96 x 96:  9.8 -> 11.0
 //   N = 3 (4096)              64 x 64: 9.1 -> 7.5      96 x 96: 10.6 -> 14.2
@@ -65,11 +65,11 @@ constexpr int pair_waves_per_simd() {
 // viscous, N = 5 (768): 16 x 16 16.6 -> 12.1, 32 x 32 15.8 -> 13.8 (more at N = 3:
 // 64 x 64 11.0 -> 12.2).
 template <int N, int SF, int FF>
-constexpr bool pair_kernel_for(int64_t E, bool viscous) {
+constexpr bool pair_kernel_for(int64_t E, bool viscous, int cus) {
   constexpr bool llf = SF == kFluxLLF && FF == kFluxLLF;
-  constexpr int kCus = 256, waves = PairShape<N>::BLOCK / 64, rounds = N == 7 ? 2 : 1;
+  constexpr int waves = PairShape<N>::BLOCK / 64, rounds = N == 7 ? 2 : 1;
   const int per_cu = viscous || !(llf || N == 7) ? 16 : 4 * pair_waves_per_simd<N, SF, FF>();
-  return E <= (int64_t)PairShape<N>::EPW * kCus * (per_cu / waves) * rounds;
+  return E <= (int64_t)PairShape<N>::EPW * cus * (per_cu / waves) * rounds;
 }
 
 // Orders the LDS accesses of one wave among its lanes.

@@ -440,7 +440,7 @@ hipError_t launch_parabolic_t(bool sc, const KParams& p, hipStream_t s) {
     }
   }
   if constexpr (NODAL) {
-    if (p.ja_box && box_table_for<DIM, N>(p.E)) {
+    if (p.ja_box && box_table_for<DIM, N>(p.E, p.cus)) {
       hipLaunchKernelGGL((viscous_flux_kernel<DIM, N, EPW, NODAL, BCS, true>), dim3((unsigned)nb),
                          dim3(BLOCK), 0, s, p);
       return hipGetLastError();

@@ -82,10 +82,10 @@ __device__ __forceinline__ const double* box_row(const KParams& p, const int* ei
 // kernel with boundaries, full arrays -> table, us a launch: N = 5 64 x 64
 // 12.3 -> 13.3, 96 x 96 21.9 -> 21.4, 128 x 128 35.8 -> 34.5; N = 3 96 x 96
 // 11.0 -> 11.7, 128 x 128 15.4 -> 14.5; periodic, table -> full arrays: N = 3
-// 96 x 96 8.6 -> 8.0).
+// 96 x 96 8.6 -> 8.0).  The line is 100 000 line threads on 256 CUs.
 template <int DIM, int N>
-constexpr bool box_table_for(int64_t E) {
-  return DIM == 3 || E * Shape<DIM, N>::LINES >= 100000;
+constexpr bool box_table_for(int64_t E, int cus) {
+  return DIM == 3 || E * Shape<DIM, N>::LINES * 256 >= (int64_t)100000 * cus;
 }
 
 // Elements per workgroup: keeps EPW * LINES near 192 threads in 3D and within one
@@ -449,7 +449,7 @@ hipError_t launch_one(const KParams& p, hipStream_t stream) {
   if constexpr (SF != kFluxAny && use_node_kernel<DIM, N, SC, BCS>())
     return launch_node_kernel<DIM, N, NODAL, SF>(p, stream);
   if constexpr (DIM == 2 && !use_node_kernel<DIM, N, SC, BCS>()) {
-    if (pair_kernel_for<N, SF, FF>(p.E, p.visc != nullptr))
+    if (pair_kernel_for<N, SF, FF>(p.E, p.visc != nullptr, p.cus))
       return launch_pair_kernel<N, SC, NODAL, SF, FF, BCS>(p, stream);
   }
   constexpr int EPW = elems_per_block<DIM, N>();
@@ -458,7 +458,7 @@ hipError_t launch_one(const KParams& p, hipStream_t stream) {
   if (nb <= 0) return hipSuccess;
   if (nb > INT32_MAX) return hipErrorInvalidValue;
   if constexpr (NODAL) {
-    if (p.ja_box && box_table_for<DIM, N>(p.E)) {
+    if (p.ja_box && box_table_for<DIM, N>(p.E, p.cus)) {
       hipLaunchKernelGGL((rhs_kernel<DIM, N, EPW, SC, NODAL, SF, FF, BCS, true>), dim3((unsigned)nb),
                          dim3(BLOCK), 0, stream, p);
       return hipGetLastError();

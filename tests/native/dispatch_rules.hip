@@ -27,3 +27,18 @@ static_assert(faces_covered<2, 1>() && faces_covered<2, 2>() && faces_covered<2,
 static_assert(faces_covered<3, 2>() && faces_covered<3, 3>() && faces_covered<3, 4>() &&
               faces_covered<3, 5>() && faces_covered<3, 7>());
 static_assert(NodeFaces<2, 7>::ROUNDS == 1 && NodeFaces<3, 7>::ROUNDS == 1);
+
+// The pair kernel takes the grids whose blocks fit the device's CUs at once and the
+// line kernel's metric table the grids above 100 000 line threads per 256 CUs,
+// whatever number of CUs the device has.
+template <int N, int F>
+constexpr bool pair_line(int64_t E, bool viscous, int cus) {
+  return pair_kernel_for<N, F, F>(E, viscous, cus) && !pair_kernel_for<N, F, F>(E + 1, viscous, cus);
+}
+static_assert(pair_line<3, kFluxLLF>(4096, false, 256) && pair_line<3, kFluxLLF>(512, false, 32));
+static_assert(pair_line<5, kFluxLLF>(1024, false, 256) && pair_line<5, kFluxLLF>(128, false, 32));
+static_assert(pair_line<7, kFluxLLF>(1024, false, 256) && pair_line<7, kFluxLLF>(512, false, 128));
+static_assert(pair_line<3, kFluxHLLC>(3072, false, 256) && pair_line<5, kFluxLLF>(96, true, 32));
+static_assert(box_table_for<2, 3>(12500, 256) && !box_table_for<2, 3>(12499, 256));
+static_assert(box_table_for<2, 3>(1563, 32) && !box_table_for<2, 3>(1562, 32));
+static_assert(box_table_for<3, 3>(1, 256) && box_table_for<3, 3>(1, 32));
