@@ -401,8 +401,9 @@ DG_HD NodePrims<DIM> face_prims(double gamma, const double* u) {
   return q;
 }
 
-// flux_llf from conservative states and their primitives, the form the
-// derivative code differentiates:
+// The LLF flux from conservative states and their primitives, as the derivatives in
+// physics_ad.hpp are written out.  The kernels evaluate flux_llf; the CPU checks hold
+// the derivatives to both.
 // 0.5 (F_L + F_R).n - 0.5 lambda (u_R - u_L), lambda = max|v.n| + max(c)|n|
 // (numerical_flux.hpp:54-68, compressible_euler3D.hpp:121-166).
 template <int DIM>
