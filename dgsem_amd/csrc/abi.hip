@@ -1,8 +1,7 @@
 // C ABI of the MI355X DGSEM right-hand side (include/dgsem_amd.h).
 //
-// The handle owns the device copies of the geometry, the neighbour table,
-// the basis tables and the per-element blending factor; state arrays belong
-// to the caller.  Everything is enqueued on the handle's stream, with no
+// The handle owns the device copies of the geometry, the basis tables and the
+// per-element blending factor; state arrays belong to the caller.  Everything is enqueued on the handle's stream, with no
 // allocation, host synchronisation or host<->device traffic inside dgsem_rhs
 // and dgsem_ssprk3_stage, so both can be captured in a HIP graph.
 #include <hip/hip_runtime.h>
@@ -62,7 +61,6 @@ void release(dgsem_handle* h) {
   hipFree(h->d_Ja);
   hipFree(h->d_invJ);
   hipFree(h->d_sn);
-  hipFree(h->d_nbr);
   hipFree(h->d_basis);
   hipFree(h->d_ja_box);
   hipFree(h->d_alpha);
@@ -79,7 +77,6 @@ void release(dgsem_handle* h) {
   h->d_ad_dgrad = h->d_ad_qbar = h->d_wq = h->d_ke_partial = nullptr;
   h->d_an_partial = h->d_ad_alpha = h->d_ad_out = h->d_fl_r = h->d_fl_w = nullptr;
   h->d_Ja = h->d_invJ = h->d_sn = h->d_basis = h->d_alpha = h->d_visc = nullptr;
-  h->d_nbr = nullptr;
   h->d_ja_box = nullptr;
 }
 
@@ -120,31 +117,6 @@ void device_geometry(const dgsem_handle* h, std::vector<double>& Ja, std::vector
   }
 }
 
-// (lower, upper) neighbour per direction: periodic wrap, or -1 at a
-// boundary face of a non-periodic direction.
-std::vector<int> neighbour_table(const dgsem::Geometry& g, const int* periodic) {
-  const int d = g.dim;
-  std::vector<int> nb(g.E * 2 * d);
-  for (int ie = 0; ie < g.cells[0]; ++ie)
-    for (int je = 0; je < g.cells[1]; ++je)
-      for (int ke = 0; ke < g.cells[2]; ++ke) {
-        const int64_t e = ((int64_t)ie * g.cells[1] + je) * g.cells[2] + ke;
-        const int id[3] = {ie, je, ke};
-        for (int r = 0; r < d; ++r)
-          for (int side = 0; side < 2; ++side) {
-            int o[3] = {id[0], id[1], id[2]};
-            o[r] += side ? 1 : -1;
-            if (!periodic[r] && (o[r] < 0 || o[r] >= g.cells[r])) {
-              nb[e * 2 * d + 2 * r + side] = -1;
-              continue;
-            }
-            o[r] = (o[r] + g.cells[r]) % g.cells[r];
-            nb[e * 2 * d + 2 * r + side] = (int)(((int64_t)o[0] * g.cells[1] + o[1]) * g.cells[2] + o[2]);
-          }
-      }
-  return nb;
-}
-
 // The table of dgsem::Operators.
 std::vector<double> basis_operators(const dgsem::BasisTables& b) {
   std::vector<double> t;
@@ -161,7 +133,6 @@ void fill_params(dgsem_handle* h) {
   p.Ja = h->d_Ja;
   p.invJ = h->d_invJ;
   p.sn = h->d_sn;
-  p.nbr = h->d_nbr;
   p.basis = h->d_basis;
   p.alpha = h->d_alpha;
   p.alpha_in = nullptr;
@@ -402,7 +373,7 @@ int dgsem_create(const dgsem_config* cfg, void* stream, dgsem_handle** out) {
   if (h->cfg.geometry == DGSEM_GEOMETRY_NODAL && h->cfg.volume_integral == DGSEM_VOLUME_SHOCK_CAPTURING)
     sn = h->geo.subcell_normals;
   if ((rc = upload(h, &h->d_Ja, Ja)) || (rc = upload(h, &h->d_invJ, invJ)) ||
-      (rc = upload(h, &h->d_sn, sn)) || (rc = upload(h, &h->d_nbr, neighbour_table(h->geo, periodic))) ||
+      (rc = upload(h, &h->d_sn, sn)) ||
       (rc = upload(h, &h->d_basis, basis_operators(h->basis))) ||
       (rc = upload(h, &h->d_alpha, std::vector<double>(4 * h->E, 0.0))) ||
       (h->cfg.equation == DGSEM_NAVIER_STOKES &&

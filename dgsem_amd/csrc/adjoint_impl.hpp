@@ -117,7 +117,7 @@ __device__ __forceinline__ bool frozen_blend(const KParams& p, int64_t e, double
   return false;
 }
 
-// Non-periodic faces (2D meshes; the neighbour table holds -1 there).  The
+// Non-periodic faces (2D meshes; face_neighbours gives -1 there).  The
 // outer state of face `face` (2 dir + upper) at boundary node bnode is the
 // one the forward's boundary_state forms (rhs_kernel_impl.hpp), with the
 // line's states read from memory.  As a map of the state it is one of

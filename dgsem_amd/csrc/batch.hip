@@ -1,7 +1,7 @@
 // Batched ensembles of independent 2D Euler cases (include/dgsem_amd.h,
 // dgsem_batch_*).  Every case keeps its own single-case handle (geometry,
-// neighbour table, basis tables, blending factor); the batch adds one state
-// arena layout, a device array of per-case kernel parameters per RK stage, a
+// basis tables, blending factor); the batch adds one state arena layout, a
+// device array of per-case kernel parameters per RK stage, a
 // cost-sorted tile list and a HIP graph of the three stage launches.
 #include <hip/hip_runtime.h>
 

@@ -23,7 +23,6 @@ struct dgsem_handle {
   double* d_Ja = nullptr;
   double* d_invJ = nullptr;
   double* d_sn = nullptr;
-  int* d_nbr = nullptr;
   double* d_basis = nullptr;  // basis operators (kernels.hpp, Operators)
   double* d_ja_box = nullptr;  // box-mesh table of the metric terms (KParams::ja_box)
   int64_t ja_box_off[3] = {0, 0, 0};
@@ -33,8 +32,9 @@ struct dgsem_handle {
   double* d_visc = nullptr;  // Navier-Stokes viscous fluxes [E][dim][var][NN]
   dgsem::KParams base{};
   // tangent / adjoint scratch, allocated on first use: d_ad_dgrad
-  // [E][dim][NV][NN] and d_ad_qbar [E][NV][NN] (Navier-Stokes), d_wq the tensor-product quadrature weight of each node, d_ke_partial the
-  // per-block sums of the kinetic-energy reduction
+  // [E][dim][NV][NN] and d_ad_qbar [E][NV][NN] (Navier-Stokes), d_wq the
+  // tensor-product quadrature weight of each node, d_ke_partial the per-block
+  // sums of the kinetic-energy reduction
   double* d_ad_dgrad = nullptr;
   double* d_ad_qbar = nullptr;
   double* d_wq = nullptr;

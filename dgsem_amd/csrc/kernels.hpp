@@ -92,10 +92,8 @@ struct KParams {
   double* out;           // L(u) or the stage result
   double c1, c2, c3;
   double floor_value;
-  const int* nbr;        // [E][2*dim] (lower, upper) neighbour per direction
-  // boundary conditions (2D): kind per face (-x, +x, -y, +y; 0 = periodic, then
-  // nbr holds -1 at that face), constant Dirichlet states and optional per-node
-  // Dirichlet states
+  // boundary conditions (2D): kind per face (-x, +x, -y, +y; 0 = periodic),
+  // constant Dirichlet states and optional per-node Dirichlet states
   int bc[6];
   double bc_state[6][5];
   const double* bc_values[6];

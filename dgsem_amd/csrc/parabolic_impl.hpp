@@ -20,8 +20,8 @@
 //     (node_kernel_for), rounded as the reference; layout [E][d][var][dof].
 // The tangent and adjoint kernels (adjoint_impl.hpp) form the gradient they
 // linearise at themselves, with line_gradient.
-// BCS (2D): some face is not periodic; the neighbour table holds -1 there and
-// the face values come from the boundary condition (wall_gradient_value and
+// BCS (2D): some face is not periodic; face_neighbours gives -1 there and the
+// face values come from the boundary condition (wall_gradient_value and
 // rhs_kernel's wall branch).
 #pragma once
 

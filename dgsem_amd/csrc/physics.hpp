@@ -4,7 +4,7 @@
 // logarithmic mean.  Expressions keep the reference's evaluation order so the
 // results agree with it to rounding.
 //
-// Reference: src/base/math_utils.hpp:8-24 (ln_mean),
+// Reference: src/base/math_utils.hpp:8-24 (the logarithmic mean),
 // src/equations/compressible_euler{2D,3D}.hpp (flux, wave speed),
 // src/base/numerical_flux.hpp:39-135,198-228 (LLF), :436-594 (Chandrashekar),
 // src/base/numerical_flux_detail.hpp:9-21.
@@ -73,19 +73,6 @@ DG_HD double div_by(double a, double b, double y) {
   (void)y;
   return a / b;
 #endif
-}
-
-// Logarithmic mean (y - x) / log(y / x) with the series branch for
-// f2 = ((x - y) / (x + y))^2 < 1e-4, math_utils.hpp:8-24.
-DG_HD double ln_mean(double x, double y) {
-  const double num = x * (x - 2.0 * y) + y * y;
-  const double den = x * (x + 2.0 * y) + y * y;
-  const double f2 = num / den;
-  if (f2 < 1.0e-4) {
-    const double poly = 2.0 + f2 * (2.0 / 3.0 + f2 * (2.0 / 5.0 + f2 * (2.0 / 7.0)));
-    return (x + y) / poly;
-  }
-  return (y - x) / log(y / x);
 }
 
 // Pressure of a conservative state.

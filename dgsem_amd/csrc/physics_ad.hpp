@@ -88,7 +88,7 @@ DG_HD void artanh_ratio_jet(double x, double y, double f2, double& Q, double& dQ
 
 // Means of the Chandrashekar flux and their partial derivatives with
 // respect to (rho_a, rho_b) and (beta_a, beta_b): rho_mean, its inverse
-// beta mean B = 1 / ln_mean(beta_a, beta_b) and p_mean = (rho_a + rho_b) /
+// beta mean B, one over the logarithmic mean of beta, and p_mean = (rho_a + rho_b) /
 // (2 (beta_a + beta_b)), as flux_chandrashekar forms them, with its branches.
 // rho_mean = s / 2 P and B = 2 Q / s; xi_x = 2 y / s^2, xi_y = -2 x / s^2.  With
 // both branches and IEEE quotients evaluated for every pair (selected without a

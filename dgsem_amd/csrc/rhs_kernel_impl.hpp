@@ -101,29 +101,14 @@ constexpr int elems_per_block() {
   return e < 1 ? 1 : e;
 }
 
-// dof of the k-th node on line `line` of direction `dir`; the line index
-// enumerates the remaining node indices in increasing dimension order.
-template <int DIM, int N>
-__device__ __forceinline__ int line_dof(int dir, int line, int k) {
-  constexpr int n = N + 1;
-  if constexpr (DIM == 2) {
-    return dir == 0 ? line * n + k : k * n + line;
-  } else {
-    const int a = line % n, b = line / n;
-    if (dir == 0) return (b * n + a) * n + k;
-    if (dir == 1) return (b * n + k) * n + a;
-    return (k * n + b) * n + a;
-  }
-}
-
-// The nodes of line `line` of direction dir: node k is dof base + k stride, at
-// the padded LDS position pbase + k pstride.  Every value is an arithmetic
-// select of the direction, so a thread sets its line up without branches;
-// per-node calls of line_dof compile to a branch each, and with the run-time
-// integer divisions of the element indices they had made up a third of the
-// 3D N = 3 kernel's instructions (with them out, and whole-node staging, the
-// SSPRK3 step at 64^3 N = 3 went from 2.34 to 2.12 ms, the warped 27 x 19 x 22
-// N = 4 right-hand side from 219 to 197 us).
+// The nodes of line `line` of direction dir (lines enumerate the remaining node
+// indices in increasing dimension order): node k is dof base + k stride, at the
+// padded LDS position pbase + k pstride.  Every value is an arithmetic select of
+// the direction, so a thread sets its line up without branches; a branch on the
+// direction for each node and the run-time integer divisions of the element
+// indices had made up a third of the 3D N = 3 kernel's instructions (with them out,
+// and whole-node staging, the SSPRK3 step at 64^3 N = 3 went from 2.34 to 2.12 ms,
+// the warped 27 x 19 x 22 N = 4 right-hand side from 219 to 197 us).
 template <int DIM, int N>
 struct LineNodes {
   int base, stride, pbase, pstride;
@@ -324,8 +309,8 @@ constexpr int min_waves_per_simd() {
 // Lower and upper face neighbours of element e along direction dir on the
 // structured grid of cells[] (element index (ie * ny + je) * nz + ke): the
 // periodic wrap, or -1 at a non-periodic boundary face (BCS: kinds from
-// p.bc) -- what the neighbour table holds, computed rather than loaded so
-// that the neighbour traces do not wait on a dependent load.  id: the
+// p.bc).  Computed rather than loaded from a table, so that the neighbour
+// traces do not wait on a dependent load.  id: the
 // element's indices (element_indices).
 template <int DIM, bool BCS>
 __device__ __forceinline__ void face_neighbours(const KParams& p, const int* id, int64_t e, int dir,
