@@ -367,8 +367,10 @@ Geometry make_geometry(const BasisTables& b, int dim, const int* cells,
 bool box_metric_table(const Geometry& g, std::vector<double>& tab, int64_t off[3]) {
   const int d = g.dim, nn = g.nn;
   const int64_t E = g.E;
-  for (int64_t i = 0; i < E * nn; ++i)
-    if (!(g.inverse_jacobian[i] > 0.0)) return false;
+  int ok = 1;
+#pragma omp parallel for schedule(static) reduction(&& : ok)
+  for (int64_t i = 0; i < E * nn; ++i) ok = ok && g.inverse_jacobian[i] > 0.0;
+  if (!ok) return false;
   auto pairs = [&](int c) -> int64_t {
     if (d == 2) return g.cells[1 - c];
     return (int64_t)g.cells[(c + 1) % 3] * g.cells[(c + 2) % 3];
@@ -394,12 +396,13 @@ bool box_metric_table(const Geometry& g, std::vector<double>& tab, int64_t off[3
   // position of node dof in a direction-r row: line * n + k, lines enumerating
   // the remaining node indices in increasing dimension order
   const int n = g.n;
-  auto line_pos = [&](int r, int dof) {
-    const int ix[3] = {dof % n, (dof / n) % n, dof / (n * n)};
-    if (d == 2) return ix[1 - r] * n + ix[r];
-    const int a = ix[r == 0 ? 1 : 0], b = ix[r == 2 ? 1 : 2];
-    return (b * n + a) * n + ix[r];
-  };
+  std::vector<int> line_pos(d * nn);
+  for (int r = 0; r < d; ++r)
+    for (int dof = 0; dof < nn; ++dof) {
+      const int ix[3] = {dof % n, (dof / n) % n, dof / (n * n)};
+      const int i0 = ix[r == 0 ? 1 : 0], i1 = d == 2 ? 0 : ix[r == 2 ? 1 : 2];
+      line_pos[r * nn + dof] = (i1 * n + i0) * n + ix[r];
+    }
   // the rows of the elements with i_c = 0
   for (int64_t e = 0; e < E; ++e) {
     int eid[3];
@@ -409,11 +412,10 @@ bool box_metric_table(const Geometry& g, std::vector<double>& tab, int64_t off[3
       const int64_t pr = pair_of(eid, c);
       for (int r = 0; r < d; ++r)
         for (int dof = 0; dof < nn; ++dof)
-          tab[off[c] + (pr * d + r) * nn + line_pos(r, dof)] = 0.5 * ja(e, dof, r, c);
+          tab[off[c] + (pr * d + r) * nn + line_pos[r * nn + dof]] = 0.5 * ja(e, dof, r, c);
     }
   }
   // every element against its rows, bit for bit
-  int ok = 1;
 #pragma omp parallel for schedule(static) reduction(&& : ok)
   for (int64_t e = 0; e < E; ++e) {
     int eid[3];
@@ -422,7 +424,8 @@ bool box_metric_table(const Geometry& g, std::vector<double>& tab, int64_t off[3
       const int64_t pr = pair_of(eid, c);
       for (int r = 0; r < d; ++r)
         for (int dof = 0; dof < nn; ++dof) {
-          const double a = 0.5 * ja(e, dof, r, c), b = tab[off[c] + (pr * d + r) * nn + line_pos(r, dof)];
+          const double a = 0.5 * ja(e, dof, r, c);
+          const double b = tab[off[c] + (pr * d + r) * nn + line_pos[r * nn + dof]];
           uint64_t ua, ub;
           std::memcpy(&ua, &a, 8);
           std::memcpy(&ub, &b, 8);
