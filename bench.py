@@ -74,7 +74,7 @@ def stage_bytes(E: int, N: int, geometry: str, box_cells=None) -> float:
 
 def read_profile(path: str) -> dict:
     """Figures of the fused kernel from a committed rocprofv3 summary: HBM
-    bytes per dispatch (FETCH_SIZE + WRITE_SIZE, calibrated), the FP64 FLOPs
+    bytes per dispatch (read requests by size + WRITE_SIZE), the FP64 FLOPs
     per dispatch counted from the FP64 VALU instruction counters, and the
     kernel's average duration in the kernel trace."""
     if not os.path.exists(path):
@@ -407,7 +407,7 @@ def main() -> int:
                     help="also time the Navier-Stokes TGV at N = 7 on 32^3 elements")
     ap.add_argument("--profile-copy-mib", type=int, default=0,
                     help="after the run, launch an elementwise copy kernel of this size "
-                         "(calibrates rocprofv3 FETCH_SIZE / WRITE_SIZE)")
+                         "(checks rocprofv3's request and WRITE_SIZE counters)")
     args = ap.parse_args()
 
     if args.cpu_baseline_child:

@@ -44,7 +44,9 @@ namespace detail {
 // Elements per workgroup, as elems_per_block: one wave in 2D (a tangent plus an
 // adjoint of a step, 192 threads -> one wave: split form N = 3 80 x 80 94 -> 80 us,
 // HLLC channel N = 3 128 x 128 209 -> 171 us, viscous N = 5 160 x 160 822 -> 725
-// us; 8% on the average of 8 x 8 to 160 x 160).
+// us; 8% on the average of 8 x 8 to 224 x 224).  A few sizes whose last round of
+// 192-thread blocks happens to be full are 1-2.5% slower (split form N = 3 160 x 160
+// 212 -> 218 us, N = 5 128 x 128 360 -> 365; before the two-kernel form 367 and 700).
 template <int DIM, int N>
 constexpr int ad_elems_per_block() {
   constexpr int e = (DIM == 2 ? 64 : 192) / Shape<DIM, N>::LINES;
@@ -80,8 +82,9 @@ __device__ __forceinline__ double sign_j(const KParams& p, int64_t e, int node) 
 }
 
 // Minimum waves per SIMD of the RHS derivative kernels: up to N = 3 the LLF
-// split-form ones fit three (168 VGPRs) with few spilled registers; the HLLC
-// and subcell derivatives would spill hundreds.
+// split-form ones are held to three (168 VGPRs; with nodal metrics at 3D N = 3 the
+// adjoint spills 14 registers, 31 with viscous terms, the tangent 83 with viscous
+// terms); the HLLC and subcell derivatives would spill hundreds.
 template <int N, bool SC, int SF>
 constexpr int ad_waves() {
   return N <= 3 && !SC && SF == kFluxLLF ? 3 : 1;
