@@ -149,9 +149,7 @@ int build_tiles(dgsem_batch* b) {
   if (e != hipSuccess) return bhip(b, e, "batch occupancy query");
   if (per_cu < 1) return bfail(b, DGSEM_E_UNSUPPORTED, "batch kernel does not fit a CU");
   const int64_t full = (int64_t)per_cu * b->num_cu;
-  int64_t g = b->grid > 0 ? b->grid : full;
-  g = std::max<int64_t>(1, std::min<int64_t>(g, b->ntiles));
-  b->grid_eff = (int)g;
+  b->grid_eff = dgsem::batch_grid(b->grid > 0 ? b->grid : full, b->ntiles, b->block);
   b->tiles_valid = true;
   drop_graph(b);
   return DGSEM_OK;

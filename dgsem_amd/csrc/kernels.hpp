@@ -224,6 +224,13 @@ struct BatchLaunch {
 // Workgroup sizes the batch kernel is built for.
 constexpr int kBatchBlocks[] = {128, 256};
 
+// Workgroups of a batch launch: as many as wanted, but no more than there are tiles
+// (the kernel strides by the grid) and than fit the 2^32 - 1 work-items of a launch.
+constexpr int batch_grid(int64_t wanted, int64_t ntiles, int block) {
+  const int64_t most = 0xffffffffll / block, g = wanted < ntiles ? wanted : ntiles;
+  return (int)(g < 1 ? 1 : (g < most ? g : most));
+}
+
 template <int BLOCK>
 hipError_t launch_batch_bs(const BatchLaunch& b, hipStream_t stream);
 hipError_t launch_batch(int block, const BatchLaunch& b, hipStream_t stream);

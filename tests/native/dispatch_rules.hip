@@ -42,3 +42,10 @@ static_assert(pair_line<3, kFluxHLLC>(3072, false, 256) && pair_line<5, kFluxLLF
 static_assert(box_table_for<2, 3>(12500, 256) && !box_table_for<2, 3>(12499, 256));
 static_assert(box_table_for<2, 3>(1563, 32) && !box_table_for<2, 3>(1562, 32));
 static_assert(box_table_for<3, 3>(1, 256) && box_table_for<3, 3>(1, 32));
+
+// A batch with a workgroup per tile stays within the work-items of a launch.
+static_assert(batch_grid(INT32_MAX, 1000, 128) == 1000 && batch_grid(512, 1000, 128) == 512);
+static_assert(batch_grid(INT32_MAX, 0, 128) == 1 && batch_grid(0, 1000, 256) == 1);
+static_assert((int64_t)batch_grid(INT32_MAX, INT32_MAX, 128) * 128 <= 0xffffffffll &&
+              batch_grid(INT32_MAX, INT32_MAX, 128) == 33554431 &&
+              batch_grid(INT32_MAX, INT32_MAX, 256) == 16777215);
